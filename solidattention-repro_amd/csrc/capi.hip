@@ -403,7 +403,7 @@ int sa_hip_consume_checksum(const float* input, int32_t elements, float* checksu
 static int lifecycle_common(const sa_paged_kv* kv, const float* k, const float* v, const uint16_t* k16,
                             const uint16_t* v16, int32_t local_tokens, int append, int32_t* status,
                             void* stream, const char* op, const float* query = nullptr,
-                            const sa_online_seal* seal = nullptr);
+                            const sa_online_seal* seal = nullptr, int32_t* arrive = nullptr);
 
 // The InfLLM online seal's arguments: a query ring that holds every token of
 // the tail (local + 32), a window >= 1, top-k within a block, one
@@ -700,7 +700,7 @@ static int decode_step_run(const sa_paged_kv* kv, const float* k, const float* v
     if (int e = check_hip(sa::launch_qkv_project(*producer, as_stream(stream)), "decode_step: q/k/v producer launch"))
       return e;
   if (!fused) {
-    if (int e = lifecycle_common(kv, k, v, k16, v16, local_tokens, 1, status, stream, op, query, seal)) return e;
+    if (int e = lifecycle_common(kv, k, v, k16, v16, local_tokens, 1, status, stream, op, query, seal, arrive)) return e;
     // few lists: the split selection (scoring spread over the device, the
     // scores after the records) where the scratch holds the scores; the same
     // ids as the one-workgroup-per-list selection
@@ -889,7 +889,8 @@ int sa_hip_local_causal_representatives(const float* prompt_queries, const uint1
 
 static int lifecycle_common(const sa_paged_kv* kv, const float* k, const float* v, const uint16_t* k16,
                             const uint16_t* v16, int32_t local_tokens, int append, int32_t* status,
-                            void* stream, const char* op, const float* query, const sa_online_seal* seal) {
+                            void* stream, const char* op, const float* query, const sa_online_seal* seal,
+                            int32_t* arrive) {
   if (int e = check_geometry(kv, op, !seal)) return e;
   if (int e = check_reps(kv, op)) return e;
   if (local_tokens < 0) return fail(SA_HIP_EINVAL, "%s: local_tokens must be >= 0", op);
@@ -929,6 +930,7 @@ static int lifecycle_common(const sa_paged_kv* kv, const float* k, const float* 
     l.ring_tokens = seal->ring_tokens;
     l.window = seal->local_window;
     l.topk = seal->topk;
+    l.arrive = arrive;
     l.seal_scale = 1.0f / sqrtf(static_cast<float>(kv->head_dim));
   }
   return check_hip(sa::launch_append_seal(l, as_stream(stream)), op);

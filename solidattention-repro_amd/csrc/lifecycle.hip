@@ -46,7 +46,7 @@ struct Params {
   int32_t group;
   int32_t local_tokens;
   int32_t append;
-  int32_t head_dim;       // D, or another multiple of 8 (append_seal_kernel<false> only)
+  int32_t head_dim;       // D, or another multiple of 8 (not the online seal)
   const float* query;     // online seal: this step's decode queries [batch][query_heads][D]
   online::Args online;
 };
@@ -57,14 +57,10 @@ __device__ inline int64_t table_page(const Params& p, int b, int64_t logical) {
   return (page >= 0 && page < p.num_pages) ? page : -1;
 }
 
-// ONLINE: keep each appended token's decode queries in the ring and seal
-// with the local-causal representative of every query head.
-template <bool ONLINE>
 __global__ __launch_bounds__(kThreads) void append_seal_kernel(const Params p) {
   const int b = blockIdx.x;
   const int tid = threadIdx.x;
   int64_t len = p.seq_len[b];
-  __shared__ float seal_smem[ONLINE ? online::kSmemFloats : 1];
 
   if (p.append) {
     const int64_t page = table_page(p, b, len / kPageTokens);
@@ -89,7 +85,6 @@ __global__ __launch_bounds__(kThreads) void append_seal_kernel(const Params p) {
       *reinterpret_cast<ushort4*>(dst + e) = kk;
       *reinterpret_cast<ushort4*>(dst + p.width + e) = vv;
     }
-    if (ONLINE) online::store_queries(p.online, p.query, b, 0, p.online.query_heads, len, tid, kThreads);
     len += 1;
     // The seal below may read the token just written by other threads.
     __syncthreads();
@@ -105,19 +100,7 @@ __global__ __launch_bounds__(kThreads) void append_seal_kernel(const Params p) {
       break;
     }
     const uint16_t* src = p.pool + page * p.page_elems;
-    if (ONLINE) {
-      // one representative per query head (rep_heads == query_heads)
-      for (int h = 0; h < p.online.query_heads; ++h) {
-        const int g = h / (p.online.query_heads / (p.width / D));
-        online::seal_head<kThreads>(p.online, b, h, src + g * D, p.token_elems, s * kPageTokens,
-                                    p.reps + (static_cast<int64_t>(b) * p.rep_heads + h) * D * p.rep_stride + s,
-                                    p.rep_stride, seal_smem);
-      }
-      ++s;
-      ++added;
-      continue;
-    }
-    const int hd = ONLINE ? D : p.head_dim;
+    const int hd = p.head_dim;
     for (int o = tid; o < p.width; o += kThreads) {  // o = kv_head * head_dim + d
       float sum = 0.0f;
 #pragma unroll 8
@@ -138,6 +121,96 @@ __global__ __launch_bounds__(kThreads) void append_seal_kernel(const Params p) {
     p.sealed[b] = static_cast<int32_t>(s);
     if (p.generation) p.generation[b] += added;
   }
+}
+
+// ---- append + InfLLM online seal ------------------------------------------------
+// Workgroup (query head h, sequence b) appends the token of h's KV head (the
+// group's workgroups write the same bytes, so that each reads only what it
+// wrote), keeps head h's query in the ring and, where the tail rule seals a
+// block, writes head h's representative of it.  A seal is a chain of
+// latencies (8-20 us a head); with one workgroup for a sequence's heads in
+// turn a step that seals took 308-326 us at 16 heads, with a workgroup per
+// head 15-16 us (4 sequences of 4-8K tokens; a step that seals nothing 4.5 us
+// either way).
+//
+// The counters move only once every workgroup of the sequence has read them:
+// the last of them to arrive at arrive[b] (zero between launches) writes
+// them, or, for a caller without counters (arrive null), online_commit_kernel
+// behind this launch.
+constexpr int kOnlineThreads = 512;
+
+// Sealed blocks after the tail rule has run on `len` tokens from block s on
+// (it stops at a block without a representative slot or a page: *full).
+__device__ inline int64_t sealed_after(const Params& p, int b, int64_t len, int64_t s, bool* full) {
+  while (len >= (s + 1) * kPageTokens + p.local_tokens) {
+    if (s >= p.rep_stride || table_page(p, b, s) < 0) {
+      *full = true;
+      break;
+    }
+    ++s;
+  }
+  return s;
+}
+
+__global__ __launch_bounds__(kOnlineThreads) void append_seal_online_kernel(const Params p, int32_t* arrive) {
+  const int h = blockIdx.x;
+  const int b = blockIdx.y;
+  const int tid = threadIdx.x;
+  __shared__ float smem[online::kSmemFloats];
+  const int64_t pos = p.seq_len[b];
+  const int64_t s0 = p.sealed[b];
+  const int64_t page = table_page(p, b, pos / kPageTokens);
+  int arrived = -1;
+  if (arrive) {
+    // the counters are in registers before this workgroup counts as arrived
+    asm volatile("" ::"s"(s0), "s"(page) : "memory");
+    if (tid == 0) arrived = __hip_atomic_fetch_add(arrive + b, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  const bool last = arrived == static_cast<int>(gridDim.x) - 1;  // (thread 0)
+  if (page < 0) {
+    if (h == 0 && tid == 0) flag_status(p.status, kStatusCapacity);
+    if (last) __hip_atomic_store(arrive + b, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return;
+  }
+  const int g = h / (p.online.query_heads / (p.width / D));
+  if (tid < kWave) {  // 4 consecutive values per lane: K in lanes 0..31, V in 32..63
+    const int is_v = tid / 32;
+    const int e = tid % 32 * 4;
+    const float4 f = *reinterpret_cast<const float4*>((is_v ? p.v : p.k) + static_cast<int64_t>(b) * p.width + g * D + e);
+    *reinterpret_cast<ushort4*>(p.pool + page * p.page_elems + (pos % kPageTokens) * p.token_elems + is_v * p.width +
+                                g * D + e) = make_ushort4(f2h_rne(f.x), f2h_rne(f.y), f2h_rne(f.z), f2h_rne(f.w));
+  }
+  online::store_queries(p.online, p.query, b, h, 1, pos, tid, kOnlineThreads);
+  __syncthreads();  // the token and its query, written by other waves, before the seal reads them
+  bool full = false;
+  const int64_t s1 = sealed_after(p, b, pos + 1, s0, &full);
+  for (int64_t s = s0; s < s1; ++s)
+    online::seal_head<kOnlineThreads>(p.online, b, h, p.pool + table_page(p, b, s) * p.page_elems + g * D,
+                                      p.token_elems, s * kPageTokens,
+                                      p.reps + (static_cast<int64_t>(b) * p.rep_heads + h) * D * p.rep_stride + s,
+                                      p.rep_stride, smem);
+  if (full && h == 0 && tid == 0) flag_status(p.status, kStatusCapacity);
+  if (last) {
+    p.seq_len[b] = static_cast<int32_t>(pos + 1);
+    p.sealed[b] = static_cast<int32_t>(s1);
+    if (p.generation) p.generation[b] += static_cast<int32_t>(s1 - s0);
+    __hip_atomic_store(arrive + b, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+}
+
+// The counters after append_seal_online_kernel without arrival counters: one
+// thread per sequence.
+__global__ __launch_bounds__(kWave) void online_commit_kernel(const Params p, int batch) {
+  const int b = blockIdx.x * kWave + threadIdx.x;
+  if (b >= batch) return;
+  const int64_t pos = p.seq_len[b];
+  if (table_page(p, b, pos / kPageTokens) < 0) return;
+  const int64_t s0 = p.sealed[b];
+  bool full = false;
+  const int64_t s1 = sealed_after(p, b, pos + 1, s0, &full);
+  p.seq_len[b] = static_cast<int32_t>(pos + 1);
+  p.sealed[b] = static_cast<int32_t>(s1);
+  if (p.generation) p.generation[b] += static_cast<int32_t>(s1 - s0);
 }
 
 // ---- bulk seal (no append): a prefill's whole pages sealed at once ----------
@@ -556,7 +629,7 @@ hipError_t launch_append_seal(const LifecycleLaunch& l, hipStream_t stream) {
     // blocks and KV heads
     if (l.ring) return hipErrorInvalidValue;
     if (l.append) {
-      hipLaunchKernelGGL(append_seal_kernel<false>, dim3(l.batch), dim3(kThreads), 0, stream, p);
+      hipLaunchKernelGGL(append_seal_kernel, dim3(l.batch), dim3(kThreads), 0, stream, p);
     } else {
       const int per_wg = kThreads / (p.head_dim / 8);  // head_dim <= 512: at least 4
       const int64_t blocks = l.table_stride < l.rep_stride ? l.table_stride : l.rep_stride;
@@ -569,7 +642,12 @@ hipError_t launch_append_seal(const LifecycleLaunch& l, hipStream_t stream) {
   } else if (l.ring) {
     p.query = l.query;
     p.online = online::Args{l.ring, l.ring_tokens, l.window, l.topk, l.query_heads, l.seal_scale};
-    hipLaunchKernelGGL(append_seal_kernel<true>, dim3(l.batch), dim3(kThreads), 0, stream, p);
+    hipLaunchKernelGGL(append_seal_online_kernel, dim3(l.query_heads, l.batch), dim3(kOnlineThreads), 0, stream, p,
+                       l.arrive);
+    if (!l.arrive) {
+      if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
+      hipLaunchKernelGGL(online_commit_kernel, dim3((l.batch + kWave - 1) / kWave), dim3(kWave), 0, stream, p, l.batch);
+    }
   } else if (!l.append) {
     // bulk seal: every block of a sequence's range in its own workgroup
     const int64_t blocks = l.table_stride < l.rep_stride ? l.table_stride : l.rep_stride;
@@ -578,7 +656,7 @@ hipError_t launch_append_seal(const LifecycleLaunch& l, hipStream_t stream) {
     if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
     hipLaunchKernelGGL(seal_commit_kernel, dim3(l.batch), dim3(kWave), 0, stream, p);
   } else {
-    hipLaunchKernelGGL(append_seal_kernel<false>, dim3(l.batch), dim3(kThreads), 0, stream, p);
+    hipLaunchKernelGGL(append_seal_kernel, dim3(l.batch), dim3(kThreads), 0, stream, p);
   }
   return hipGetLastError();
 }

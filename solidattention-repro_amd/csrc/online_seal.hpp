@@ -60,6 +60,8 @@ __device__ inline void store_queries(const Args& a, const float* query, int b, i
 // first_pos: the position of the block's token 0; rep: the representative's
 // value of d = 0 (d at rep + d * rep_stride).  Every thread of the workgroup
 // calls it (workgroup barriers inside); smem: kSmemFloats floats of LDS.
+// Bound by its chain of latencies (two loads' round trips, the 128-step dots,
+// then folds over 32 entries between barriers), not by bytes or arithmetic.
 template <int kThreads>
 __device__ inline void seal_head(const Args& a, int b, int h, const uint16_t* keys, int64_t token_elems,
                                  int64_t first_pos, float* rep, int64_t rep_stride, float* smem) {
@@ -72,27 +74,56 @@ __device__ inline void seal_head(const Args& a, int b, int h, const uint16_t* ke
   int* order = reinterpret_cast<int*>(row + kT);                        // [32]
 
   const float* ring_h = a.ring + (static_cast<int64_t>(b) * a.query_heads + h) * a.ring_tokens * kDim;
-  for (int e = tid; e < kT * kDim; e += kThreads) {
-    const int t = e / kDim;
-    const int d = e % kDim;
-    qs[t * kQStride + d] = ring_h[((first_pos + t) % a.ring_tokens) * kDim + d];
+  // every load of the queries and keys is issued before the first is used
+  constexpr int kQLoads = kT * kDim / kThreads;
+  constexpr int kKLoads = kT * kDim / 2 / kThreads;
+  const int slot0 = static_cast<int>(first_pos % a.ring_tokens);
+  float qv[kQLoads];
+  uint32_t kv[kKLoads];
+#pragma unroll
+  for (int i = 0; i < kQLoads; ++i) {
+    const int e = tid + i * kThreads;
+    int slot = slot0 + e / kDim;  // the ring holds the whole block: at most one wrap
+    if (slot >= a.ring_tokens) slot -= a.ring_tokens;
+    qv[i] = ring_h[static_cast<int64_t>(slot) * kDim + e % kDim];
   }
-  for (int e = tid; e < kT * kDim / 2; e += kThreads) {
-    const int t = e / (kDim / 2);
-    const int w = e % (kDim / 2);
-    ks[t * kKStride + w] = *reinterpret_cast<const uint32_t*>(keys + t * token_elems + 2 * w);
+#pragma unroll
+  for (int i = 0; i < kKLoads; ++i) {
+    const int e = tid + i * kThreads;
+    kv[i] = *reinterpret_cast<const uint32_t*>(keys + e / (kDim / 2) * token_elems + 2 * (e % (kDim / 2)));
+  }
+#pragma unroll
+  for (int i = 0; i < kQLoads; ++i) {
+    const int e = tid + i * kThreads;
+    qs[e / kDim * kQStride + e % kDim] = qv[i];
+  }
+#pragma unroll
+  for (int i = 0; i < kKLoads; ++i) {
+    const int e = tid + i * kThreads;
+    ks[e / (kDim / 2) * kKStride + e % (kDim / 2)] = kv[i];
   }
   __syncthreads();
 
+  // Pairs (query i, key j <= i): rows r and 31 - r together hold 33 of them,
+  // so the 528 pairs are numbered with no gaps (a 32 x 32 grid would leave
+  // half the lanes without a pair).
+  auto pair = [](int e, int& i, int& j) {
+    const int r = e / (kT + 1);
+    const int c = e % (kT + 1);
+    i = c <= r ? r : kT - 1 - r;
+    j = c <= r ? c : c - r - 1;
+  };
+  constexpr int kPairs = kT * (kT + 1) / 2;
+
   // logits of query i over keys j in [i + 1 - window, i] (selection.cpp:36-48)
-  for (int e = tid; e < kT * kT; e += kThreads) {
-    const int i = e / kT;
-    const int j = e % kT;
-    if (j > i || i - j >= a.window) continue;
+  for (int e = tid; e < kPairs; e += kThreads) {
+    int i, j;
+    pair(e, i, j);
+    if (i - j >= a.window) continue;
     const float* q = qs + i * kQStride;
     const uint32_t* k = ks + j * kKStride;
     float dot = 0.0f;
-#pragma unroll 8
+#pragma unroll 16
     for (int w = 0; w < kDim / 2; ++w) {
       const uint32_t kw = k[w];
       dot = dot + q[2 * w] * lo_h2f(kw);
@@ -101,53 +132,73 @@ __device__ inline void seal_head(const Args& a, int b, int h, const uint16_t* ke
     ls[i * kLStride + j] = dot * a.scale;
   }
   __syncthreads();
+  // The serial folds over a row or column of logits read all 32 entries first
+  // (LDS reads in flight together) and skip those outside the window.  Each
+  // fold's row index is opaque to the compiler, which would otherwise keep 32
+  // lane masks from one fold to the next in scalar registers.
+  const uint32_t window = static_cast<uint32_t>(a.window);
+  auto in_window = [window](int back) { return static_cast<uint32_t>(back) < window; };  // 0 <= back < window
+  auto opaque = [](int x) {
+    asm("" : "+v"(x));
+    return x;
+  };
   if (tid < kT) {
-    const int i = tid;
-    const int start = i + 1 > a.window ? i + 1 - a.window : 0;
+    const int i = opaque(tid);
+    float x[kT];
+#pragma unroll
+    for (int j = 0; j < kT; ++j) x[j] = ls[i * kLStride + j];
     float maximum = -__builtin_huge_valf();
-    for (int j = start; j <= i; ++j) maximum = fmaxf(maximum, ls[i * kLStride + j]);
+#pragma unroll
+    for (int j = 0; j < kT; ++j) maximum = in_window(i - j) ? fmaxf(maximum, x[j]) : maximum;
     row[i] = maximum;
   }
   __syncthreads();
   // exponentials (selection.cpp:51-52)
-  for (int e = tid; e < kT * kT; e += kThreads) {
-    const int i = e / kT;
-    const int j = e % kT;
-    if (j > i || i - j >= a.window) continue;
+  for (int e = tid; e < kPairs; e += kThreads) {
+    int i, j;
+    pair(e, i, j);
+    if (i - j >= a.window) continue;
     ls[i * kLStride + j] = expf_glibc(ls[i * kLStride + j] - row[i]);
   }
   __syncthreads();
   if (tid < kT) {  // denominators in key order (selection.cpp:53)
-    const int i = tid;
-    const int start = i + 1 > a.window ? i + 1 - a.window : 0;
+    const int i = opaque(tid);
+    float x[kT];
+#pragma unroll
+    for (int j = 0; j < kT; ++j) x[j] = ls[i * kLStride + j];
     float denominator = 0.0f;
-    for (int j = start; j <= i; ++j) denominator = denominator + ls[i * kLStride + j];
+#pragma unroll
+    for (int j = 0; j < kT; ++j) denominator = in_window(i - j) ? denominator + x[j] : denominator;
     row[i] = denominator;
   }
   __syncthreads();
-  for (int e = tid; e < kT * kT; e += kThreads) {
-    const int i = e / kT;
-    const int j = e % kT;
-    if (j > i || i - j >= a.window) continue;
+  for (int e = tid; e < kPairs; e += kThreads) {
+    int i, j;
+    pair(e, i, j);
+    if (i - j >= a.window) continue;
     ls[i * kLStride + j] = ls[i * kLStride + j] / row[i];
   }
   __syncthreads();
   if (tid < kT) {  // the mass key j received, in query order (selection.cpp:55-58)
-    const int j = tid;
-    const int last = j + a.window - 1 < kT - 1 ? j + a.window - 1 : kT - 1;
+    const int j = opaque(tid);
+    float x[kT];
+#pragma unroll
+    for (int i = 0; i < kT; ++i) x[i] = ls[i * kLStride + j];
     float r = 0.0f;
-    for (int i = j; i <= last; ++i) r = r + ls[i * kLStride + j];
+#pragma unroll
+    for (int i = 0; i < kT; ++i) r = in_window(i - j) ? r + x[i] : r;
     received[j] = r;
   }
   __syncthreads();
   if (tid < kT) {  // stable descending rank (selection.cpp:71-76)
     const int j = tid;
     const float rj = received[j];
+    float x[kT];
+#pragma unroll
+    for (int k = 0; k < kT; ++k) x[k] = received[k];
     int rank = 0;
-    for (int k = 0; k < kT; ++k) {
-      const float rk = received[k];
-      rank += (mass_before(rk, rj) || (k < j && mass_tied(rk, rj))) ? 1 : 0;
-    }
+#pragma unroll
+    for (int k = 0; k < kT; ++k) rank += (mass_before(x[k], rj) || (k < j && mass_tied(x[k], rj))) ? 1 : 0;
     order[rank] = j;
   }
   __syncthreads();

@@ -277,6 +277,7 @@ struct LifecycleLaunch {
   int32_t window;
   int32_t topk;
   float seal_scale;
+  int32_t* arrive;  // online seal: [batch] zeroed arrival counters, left at zero (null: one launch more)
 };
 
 hipError_t launch_append_seal(const LifecycleLaunch& l, hipStream_t stream);
