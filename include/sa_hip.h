@@ -316,7 +316,11 @@ int sa_hip_select_attend(const sa_paged_kv* kv, const float* query,
  * to 256 bytes) followed by the attention's split records (padded to 256
  * bytes) and the split selection's scores (batch x query_heads x rep_stride
  * floats; used when the step runs as separate launches with few lists, and
- * at every head_dim other than 128).  The caller
+ * at every head_dim other than 128), and at least as large as the counters
+ * and the partial records of a one-launch step that spreads each list over
+ * several workgroups.  A smaller workspace that holds the counters, the
+ * split records and the scores is accepted (with fewer workgroups per list,
+ * or separate launches).  The caller
  * zeroes it ONCE before the first call; every call leaves the counters at
  * zero again.  Calls sharing a workspace must not run concurrently. */
 size_t sa_hip_decode_step_workspace_bytes(const sa_paged_kv* kv,
@@ -332,7 +336,11 @@ size_t sa_hip_decode_step_workspace_bytes(const sa_paged_kv* kv,
  * workgroup), then scores, selects and attends; the last workgroup of a
  * sequence to arrive writes its counters.  The online seal (the _online
  * variant) runs as one launch only with select_groups == kv_heads.
- * Otherwise it runs the three launches.  The _f16 variant takes raw FP16
+ * Otherwise, with few enough sequences and short enough lists, it is still
+ * one launch (behind append + seal for the online seal) with several
+ * workgroups per (sequence, KV head), however many the device has room for;
+ * splits only selects this form (ids and state the same, outputs to fp32
+ * rounding).  Else it runs the separate launches.  The _f16 variant takes raw FP16
  * K/V bits like sa_hip_append_seal_f16.  Replaces the reference's per-layer
  * decode sequence of append_fp16_kv (qwen_layer_main.cpp:270-281 via
  * qwen_chain_main.cpp:390-391), the tail seal (kv_lifecycle_main.cpp:92-113),

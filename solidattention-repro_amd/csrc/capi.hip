@@ -642,9 +642,37 @@ static size_t split_scores_bytes(const sa_paged_kv* kv, int32_t select_groups) {
   return static_cast<size_t>(kv->batch) * select_groups * (kv->rep_stride > 0 ? kv->rep_stride : 0) * sizeof(float);
 }
 
+// What every step accepts (counters, the caller's split records, scores); the
+// workspace is sized for the records of the split step as well, which uses as
+// many splits as the workspace holds records for.
+static size_t step_min_bytes(const sa_paged_kv* kv, int32_t splits) {
+  return arrive_bytes(kv->batch) + split_records_bytes(kv, splits) + split_scores_bytes(kv, kv->query_heads);
+}
+
+static size_t split_step_bytes(const sa_paged_kv* kv, int32_t splits) {
+  return static_cast<size_t>(kv->batch) * kv->query_heads * splits * sa::part_stride(kv->head_dim) * sizeof(float);
+}
+
 size_t sa_hip_decode_step_workspace_bytes(const sa_paged_kv* kv, int32_t splits) {
   if (!kv || kv->batch <= 0) return 0;
-  return arrive_bytes(kv->batch) + split_records_bytes(kv, splits) + split_scores_bytes(kv, kv->query_heads);
+  const size_t need = step_min_bytes(kv, splits);
+  if (kv->kv_heads <= 0 || kv->query_heads <= 0 || kv->head_dim <= 0) return need;
+  const int32_t cap = sa::split_step_cap(kv->batch, kv->query_heads, kv->kv_heads, kv->head_dim);
+  return std::max(need, arrive_bytes(kv->batch) + split_step_bytes(kv, cap));
+}
+
+// The step with several workgroups per list, where it applies and the records
+// fit (*done): one launch, or, with the online seal (f.append 0 by then), the
+// launch behind append + seal.
+static int try_split_step(const sa_paged_kv* kv, const sa::SelectAttendLaunch& f, void* records,
+                          size_t records_bytes, void* stream, bool* done) {
+  *done = false;
+  int32_t s = sa::split_step_splits(f);
+  while (s > 0 && split_step_bytes(kv, s) > records_bytes) --s;
+  if (s < 1) return SA_HIP_OK;
+  *done = true;
+  return check_hip(sa::launch_split_step(f, static_cast<float*>(records), s, as_stream(stream)),
+                   "decode_step launch");
 }
 
 // The decode step on explicit scratch: `arrive` holds kv->batch arrival
@@ -676,11 +704,27 @@ static int decode_step_run(const sa_paged_kv* kv, const float* k, const float* v
   if (producer && (seal || k16 || sa::general_head_dim(kv->head_dim)))
     return fail(SA_HIP_EINVAL, "%s: the q/k/v producer feeds head_dim %d and fp32 tokens, without the online seal",
                 op, sa::kHeadDim);
+  auto step_launch = [&] {
+    sa::SelectAttendLaunch f = fused_launch(kv, l, scale, out);
+    f.append = 1;
+    f.local_tokens = local_tokens;
+    f.k = k;
+    f.v = v;
+    f.k16 = k16;
+    f.v16 = v16;
+    f.arrive = arrive;
+    return f;
+  };
   if (sa::general_head_dim(kv->head_dim) && (seal || !sa_hip_select_attend_fused(kv, params, splits))) {
     // the general kernels in sequence (where the one-launch step does not
     // apply): append + seal, scoring into the workspace's scores, selection,
     // attention
     if (seal) return fail(SA_HIP_EINVAL, "%s: the online seal is built for head_dim %d", op, sa::kHeadDim);
+    if (!clear_arrive) {
+      bool done = false;
+      const int e = try_split_step(kv, step_launch(), records, records_bytes, stream, &done);
+      if (e || done) return e;
+    }
     const size_t rb = split_records_bytes(kv, splits);
     const size_t sb = split_scores_bytes(kv, params->select_groups);
     if (records_bytes < rb + sb)
@@ -700,7 +744,18 @@ static int decode_step_run(const sa_paged_kv* kv, const float* k, const float* v
     if (int e = check_hip(sa::launch_qkv_project(*producer, as_stream(stream)), "decode_step: q/k/v producer launch"))
       return e;
   if (!fused) {
+    sa::SelectAttendLaunch f = step_launch();
+    bool done = false;
+    if (!seal && !clear_arrive) {
+      const int e = try_split_step(kv, f, records, records_bytes, stream, &done);
+      if (e || done) return e;
+    }
     if (int e = lifecycle_common(kv, k, v, k16, v16, local_tokens, 1, status, stream, op, query, seal, arrive)) return e;
+    if (seal && !clear_arrive) {
+      f.append = 0;
+      const int e = try_split_step(kv, f, records, records_bytes, stream, &done);
+      if (e || done) return e;
+    }
     // few lists: the split selection (scoring spread over the device, the
     // scores after the records) where the scratch holds the scores; the same
     // ids as the one-workgroup-per-list selection
@@ -716,14 +771,15 @@ static int decode_step_run(const sa_paged_kv* kv, const float* k, const float* v
     return attention_common(kv, query, selected, counts, params->select_groups, params->sel_stride, scale, out,
                             records, records_bytes, splits, status, stream, 0);
   }
-  sa::SelectAttendLaunch f = fused_launch(kv, l, scale, out);
-  f.append = 1;
-  f.local_tokens = local_tokens;
-  f.k = k;
-  f.v = v;
-  f.k16 = k16;
-  f.v16 = v16;
-  f.arrive = arrive;
+  sa::SelectAttendLaunch f = step_launch();
+  if (!clear_arrive && !seal && params->select_groups != kv->kv_heads) {
+    // the shared selection's few workgroups, each list split over several
+    bool done = false;
+    if (sa::split_step_splits(f) > 1) {
+      const int e = try_split_step(kv, f, records, records_bytes, stream, &done);
+      if (e || done) return e;
+    }
+  }
   if (seal) {
     f.ring = seal->query_ring;
     f.ring_tokens = seal->ring_tokens;
@@ -754,7 +810,7 @@ static int decode_step_common(const sa_paged_kv* kv, const float* k, const float
                               float* out, void* workspace, size_t workspace_bytes, int32_t splits, int32_t* status,
                               void* stream, const char* op, const sa::QkvLaunch* producer = nullptr) {
   if (!kv || kv->batch <= 0) return fail(SA_HIP_EINVAL, "%s: null sa_paged_kv or empty batch", op);
-  const size_t need = sa_hip_decode_step_workspace_bytes(kv, splits);
+  const size_t need = step_min_bytes(kv, splits);
   if (!workspace || workspace_bytes < need)
     return fail(SA_HIP_EINVAL, "%s: workspace of %zu bytes needed, %zu given", op, need, workspace_bytes);
   if (!aligned16(workspace)) return fail(SA_HIP_EINVAL, "%s: workspace must be 16-byte aligned", op);
@@ -788,7 +844,7 @@ int sa_hip_decode_step_online(const sa_paged_kv* kv, const float* k, const float
   const char* op = "decode_step_online";
   if (!seal) return fail(SA_HIP_EINVAL, "%s: null online seal", op);
   if (!kv || kv->batch <= 0) return fail(SA_HIP_EINVAL, "%s: null sa_paged_kv or empty batch", op);
-  const size_t need = sa_hip_decode_step_workspace_bytes(kv, splits);
+  const size_t need = step_min_bytes(kv, splits);
   if (!workspace || workspace_bytes < need)
     return fail(SA_HIP_EINVAL, "%s: workspace of %zu bytes needed, %zu given", op, need, workspace_bytes);
   if (!aligned16(workspace)) return fail(SA_HIP_EINVAL, "%s: workspace must be 16-byte aligned", op);

@@ -197,6 +197,16 @@ struct SelectAttendLaunch {
 bool select_attend_supported(int32_t query_heads, int32_t kv_heads, int32_t select_groups, int32_t sel_stride,
                              const float* reps, int32_t rep_stride);
 int select_attend_per_cu(int32_t query_heads, int32_t kv_heads);
+// The step with several workgroups per (sequence, KV head), for fewer lists
+// than the device has workgroup slots; one launch whose last workgroups merge
+// the partial records (query_heads / kv_heads * part_stride(head_dim) floats
+// per workgroup).  cap: the most splits any call of this geometry uses (sizes
+// the workspace); splits: this call's, 0 where the step does not apply.
+int32_t split_step_cap(int32_t batch, int32_t query_heads, int32_t kv_heads, int32_t head_dim);
+int32_t split_step_splits(const SelectAttendLaunch& s);
+// s.append 0: the token is already appended and sealed.  s.arrive as for the
+// one-launch step.
+hipError_t launch_split_step(const SelectAttendLaunch& s, float* records, int32_t splits, hipStream_t stream);
 // The one-launch form of the shared selection (select_groups 1 over several
 // KV heads): 1, 2 or 4 query heads per KV head, representatives per KV head,
 // rep_stride <= kMaxSharedFusedBlocks, and the representatives read once per

@@ -71,6 +71,11 @@ struct Params {
   int32_t local_tokens;
   float qscale;  // softmax scale * log2(e)
   online::Args online;  // InfLLM online seal (ring non-null)
+  // split launches: `splits` workgroups per (sequence, KV head), their partial
+  // records, and the width of a KV head's field in arrive[b]
+  float* part;
+  int32_t splits;
+  int32_t field_bits;
 };
 
 __device__ inline int64_t table_page(const attn::PoolView& v, int b, int64_t logical) {
@@ -184,6 +189,122 @@ __device__ inline void commit_sequence(const Params& p, int b, int64_t len, int 
   p.arrive[b] = 0;
 }
 
+// ---- several workgroups per (sequence, KV head) -------------------------------
+// With fewer lists than the device has workgroup slots, `splits` workgroups
+// share one list: each appends, scores and selects for itself (the same bytes
+// and ids; the representatives' later reads come from the L2, since with
+// kv_heads a multiple of 8 a list's workgroups land on one XCD) and attends its
+// share of the pages.  Partial records (max, sum, accumulator) meet in the
+// workspace and the last workgroup of the list merges them in split order.
+//
+// One counter per sequence counts all of its workgroups: KV head g's field of
+// field_bits bits at bit g * field_bits (32 bits hold kv_heads fields that
+// count to `splits`, see split_field_bits()).  The last workgroup of the
+// sequence clears it and, for a step that appends, writes the sequence
+// counters: every other workgroup has read them by then.
+//
+// Bound by latency (a chain of loads, dots, a selection and a page or two per
+// wave) rather than bytes, and before by launches: append + seal, scoring,
+// selection, attention and merge cost about 4.5 us each even with nothing to
+// do.  Per layer, as those launches and as this one: 16 sequences of 4-8K
+// tokens, 16/8 heads 51 -> 35 us; 16 x 8-16K, 64/8 heads 62 -> 54 us; 32 x
+// 5-10K, 16/8 heads of 64: 59 -> 42 us; 4 x 4-8K with online
+// representatives (append + seal in its own launch) 54 -> 38 us.
+struct SplitEnd {
+  bool list_last;
+  bool seq_last;
+};
+
+// Every thread calls it, its record stores issued.
+__device__ inline SplitEnd split_arrive(const Params& p, int b, int g, uint32_t* s_old) {
+  __builtin_amdgcn_s_waitcnt(0);  // this thread's record stores have completed
+  __syncthreads();
+  const uint32_t unit = 1u << (g * p.field_bits);
+  if (threadIdx.x == 0)
+    *s_old = __hip_atomic_fetch_add(reinterpret_cast<uint32_t*>(p.arrive) + b, unit, __ATOMIC_RELAXED,
+                                    __HIP_MEMORY_SCOPE_AGENT);
+  __syncthreads();
+  const uint32_t now = *s_old + unit;
+  const uint32_t mask = (1u << p.field_bits) - 1u;
+  uint32_t full = 0;
+  for (int h = 0; h < p.v.kv_heads; ++h) full |= static_cast<uint32_t>(p.splits) << (h * p.field_bits);
+  return SplitEnd{((now >> (g * p.field_bits)) & mask) == static_cast<uint32_t>(p.splits), now == full};
+}
+
+// This workgroup's record of (sequence b, KV head g, split z, head h).
+__device__ inline float* split_record(const Params& p, int b, int g, int z, int G, int h, int hd) {
+  return p.part + (((static_cast<int64_t>(b) * p.v.kv_heads + g) * p.splits + z) * G + h) * part_stride(hd);
+}
+
+__device__ inline void store_record(float* rec, int d, float mx, float lw, float aw) {
+  if (d == 0) {
+    store_agent(rec, mx);
+    store_agent(rec + 1, lw);
+  }
+  store_agent(rec + kPartPad + d, aw);
+}
+
+// The list's records merged (log-sum-exp, in split order) into its G output
+// rows of hd values; the loads of all records of a batch are in flight
+// together.
+constexpr int kMaxStepSplits = 16;
+
+template <int G>
+__device__ inline void merge_split_records(const Params& p, int b, int g, int hd) {
+  constexpr int kBatch = 8;
+  for (int o = threadIdx.x; o < G * hd; o += kThreads) {
+    const int h = o / hd;
+    const int d = o % hd;
+    const float* rec = split_record(p, b, g, 0, G, h, hd);
+    const int64_t rstride = static_cast<int64_t>(G) * part_stride(hd);
+    float mx = attn::kNegInf, lw = 0.0f, aw = 0.0f;
+    for (int z0 = 0; z0 < p.splits; z0 += kBatch) {
+      float m[kBatch], l[kBatch], a[kBatch];
+#pragma unroll
+      for (int j = 0; j < kBatch; ++j) {
+        const float* r = rec + min(z0 + j, p.splits - 1) * rstride;
+        m[j] = load_agent(r);
+        l[j] = load_agent(r + 1);
+        a[j] = load_agent(r + kPartPad + d);
+      }
+      float bm = mx;
+#pragma unroll
+      for (int j = 0; j < kBatch; ++j) bm = fmaxf(bm, m[j]);
+      if (bm == attn::kNegInf) continue;
+      const float corr = __builtin_amdgcn_exp2f(mx - bm);  // (nothing so far: exp2(-inf) = 0)
+      lw *= corr;
+      aw *= corr;
+      mx = bm;
+#pragma unroll
+      for (int j = 0; j < kBatch; ++j) {
+        if (z0 + j >= p.splits || m[j] == attn::kNegInf) continue;
+        const float f = __builtin_amdgcn_exp2f(m[j] - mx);
+        lw = __builtin_fmaf(l[j], f, lw);
+        aw = __builtin_fmaf(a[j], f, aw);
+      }
+    }
+    p.out[(static_cast<int64_t>(b) * p.query_heads + g * G + h) * hd + d] = lw > 0.0f ? aw / lw : 0.0f;
+  }
+}
+
+// After the workgroup's record stores: the last workgroup of the list merges,
+// the last of the sequence clears the counter and commits an append.
+template <int G, bool APPEND>
+__device__ inline void finish_split(const Params& p, int b, int g, int hd, int64_t len, int n, const SeqCommit& c,
+                                    uint32_t* s_old) {
+  const SplitEnd e = split_arrive(p, b, g, s_old);
+  if (!e.list_last) return;
+  merge_split_records<G>(p, b, g, hd);
+  if (e.seq_last && threadIdx.x == 0) {
+    if (APPEND && c.appended) {
+      p.seq_len[b] = static_cast<int32_t>(len);
+      p.sealed[b] = n;
+      if (p.generation) p.generation[b] = c.gen + c.added;
+    }
+    p.arrive[b] = 0;
+  }
+}
+
 // ---- the planned page walk (both fused kernels) ------------------------------
 // After the scoring every wave walks its own positions of one list:
 //   * positions [0, F): the forced blocks (init, then local: selected
@@ -292,7 +413,9 @@ __device__ inline void list_late(const Params& p, int b, ClaimSmem& cl, int32_t*
 }
 
 // Page source of the walk: this wave's planned positions (see above); all
-// values wave-uniform.
+// values wave-uniform.  SPLIT: the positions are planned over the waves of
+// the list's p.splits workgroups (each with its own wave 0, which selects).
+template <bool SPLIT>
 struct PlanPages {
   ClaimSmem& cs;
   const int32_t* late;
@@ -302,15 +425,45 @@ struct PlanPages {
   int F;        // forced positions listed early
   int n;        // sealed blocks
   int64_t len;  // tokens (after this step's append)
+  int z;        // this workgroup of the list's `splits`
+  int splits;
   int e_next;   // next forced position of this wave (F when done)
   int l_next = 0;
   int l_end = 0;
   bool ready = false;
 
   __device__ PlanPages(ClaimSmem& cs_, const int32_t* late_, const attn::PoolView& v_, int b_, int wave_, int F_,
-                       int n_, int64_t len_)
-      : cs(cs_), late(late_), v(v_), b(b_), wave(wave_), F(F_), n(n_), len(len_) {
-    e_next = wave == 0 ? F : wave - 1;
+                       int n_, int64_t len_, int z_ = 0, int splits_ = 1)
+      : cs(cs_), late(late_), v(v_), b(b_), wave(wave_), F(F_), n(n_), len(len_), z(SPLIT ? z_ : 0),
+        splits(SPLIT ? splits_ : 1) {
+    e_next = wave == 0 ? F : (wave - 1) * splits + z;
+    if (e_next > F) e_next = F;
+  }
+
+  // The split plan: walker u = wave * splits + z of 8 * splits (<= 128), the
+  // selecting waves first; the same balance as below, each lane planning two
+  // walkers and a prefix sum giving where a walker's range begins.
+  __device__ inline int split_want(int u, int late_n) const {
+    const int walkers = kWaves * splits;
+    if (u >= walkers) return 0;
+    const int total = F + late_n + kSelectPages * splits;
+    const int target = total / walkers + (u < total % walkers ? 1 : 0);
+    const int r = u - splits;  // rank among the forced positions' walkers
+    const int step = (kWaves - 1) * splits;
+    const int want = target - (r < 0 ? kSelectPages : (r < F ? (F - r + step - 1) / step : 0));
+    return want > 0 ? want : 0;
+  }
+  __device__ inline void plan_late_split(int late_n) {
+    const int lane = threadIdx.x % kWave;
+    const int lo = split_want(2 * lane, late_n), hi = split_want(2 * lane + 1, late_n);
+    const int before = static_cast<int>(wave_prefix_sum(static_cast<uint32_t>(lo + hi))) - lo - hi;
+    const int u = __builtin_amdgcn_readfirstlane(wave * splits + z);
+    int begin = __builtin_amdgcn_readlane(before, u >> 1);
+    const int first = __builtin_amdgcn_readlane(lo, u >> 1), second = __builtin_amdgcn_readlane(hi, u >> 1);
+    if (u & 1) begin += first;
+    const int end = begin + ((u & 1) ? second : first);
+    l_next = begin < late_n ? begin : late_n;
+    l_end = u == kWaves * splits - 1 ? late_n : (end < late_n ? end : late_n);
   }
 
   // Forced positions of wave w (>= 1): w - 1, w - 1 + 7, ... below F.
@@ -342,7 +495,7 @@ struct PlanPages {
   __device__ inline attn::PageRef next(bool wait) {
     while (e_next < F) {
       const int c = e_next;
-      e_next += kWaves - 1;
+      e_next += (kWaves - 1) * splits;
       const int32_t page = __builtin_amdgcn_readfirstlane(cs.early[c]);
       if (page >= 0) return attn::PageRef{page, kPageTokens};
     }
@@ -351,7 +504,8 @@ struct PlanPages {
         return attn::PageRef{0, -1};
       wait_late(cs);
       ready = true;
-      plan_late(__builtin_amdgcn_readfirstlane(cs.late_n));
+      if constexpr (SPLIT) plan_late_split(__builtin_amdgcn_readfirstlane(cs.late_n));
+      else plan_late(__builtin_amdgcn_readfirstlane(cs.late_n));
     }
     const int mid = __builtin_amdgcn_readfirstlane(cs.late_mid);
     const int tail_listed = __builtin_amdgcn_readfirstlane(cs.tail_listed);
@@ -385,12 +539,15 @@ struct NoProducer {};
 // wave 1 KV head g's k (lanes 0..31) and v (lanes 32..63), the layout in which
 // wave 1 appends the token.  q, k and v are also written out, the values the
 // producer's reduce launch would write.
-template <int G, int GR, bool APPEND, bool F16, bool ONLINE, class Prod>
+// SPLIT: p.splits workgroups (blockIdx.z) share the list (see above).
+template <int G, int GR, bool APPEND, bool F16, bool ONLINE, bool SPLIT, class Prod>
 __device__ inline void decode_body(const Params& p, const Prod& qp) {
   constexpr bool kProd = !std::is_same<Prod, NoProducer>::value;
   static_assert(!kProd || (G <= 2 && APPEND && !F16 && !ONLINE), "the producer epilogue: 1-2 heads, fp32 token");
+  static_assert(!SPLIT || !ONLINE, "the workgroups of a list would all run its online seal");
   const int g = blockIdx.x;
   const int b = blockIdx.y;
+  const int z = SPLIT ? blockIdx.z : 0;
   const int tid = threadIdx.x;
   const int wave = tid / kWave;
   const int lane = tid % kWave;
@@ -400,6 +557,7 @@ __device__ inline void decode_body(const Params& p, const Prod& qp) {
   __shared__ uint32_t hist[256];
   __shared__ attn::CombineSmem<G, kWaves> cs;
   __shared__ ClaimSmem cl;
+  __shared__ uint32_t s_old;  // (SPLIT)
 
   const int64_t out_row = static_cast<int64_t>(b) * p.v.kv_heads + g;
   // the group's query rows, loaded at entry (their latency overlaps the append)
@@ -457,7 +615,7 @@ __device__ inline void decode_body(const Params& p, const Prod& qp) {
     commit.gen = p.generation ? p.generation[b] : 0;
     commit.appended = append_seal_head<G, F16, ONLINE, kProd>(p, b, g, len, n, commit.added,
                                                               reinterpret_cast<float*>(keys), tok);
-    if (tid == 0) commit.arrived = atomicAdd(&p.arrive[b], 1);
+    if (!SPLIT && tid == 0) commit.arrived = atomicAdd(&p.arrive[b], 1);
   }
 
   attn::WaveState<G> st;
@@ -503,15 +661,16 @@ __device__ inline void decode_body(const Params& p, const Prod& qp) {
     if (!n_ok || bs.bad) {
       if (lane == 0) {
         flag_status(p.v.status, n_ok ? kStatusBadBudget : kStatusCapacity);
-        p.counts[out_row] = 0;
+        if (z == 0) p.counts[out_row] = 0;
       }
     } else {
-      count = sel::select_ids_wave(keys, n, bs, hist, p.selected + out_row * p.sel_stride, p.sel_stride, late);
-      if (lane == 0) p.counts[out_row] = count;
+      count = sel::select_ids_wave(keys, n, bs, hist, z == 0 ? p.selected + out_row * p.sel_stride : nullptr,
+                                   p.sel_stride, late);
+      if (lane == 0 && z == 0) p.counts[out_row] = count;
     }
     list_late(p, b, cl, late, kMaxSelectBlocks, count, fb, wn, tail_pages, lane);
   }
-  PlanPages src(cl, late, p.v, b, wave, fb.F, wn, wlen);
+  PlanPages<SPLIT> src(cl, late, p.v, b, wave, fb.F, wn, wlen, z, p.splits);
   for (;;) {
     const attn::PageRef pr = src.next(true);
     if (pr.valid <= 0) break;
@@ -526,22 +685,29 @@ __device__ inline void decode_body(const Params& p, const Prod& qp) {
     const int d = o % D;
     float mx, lw, aw;
     attn::combine_element<G, kWaves>(cs, h, d, mx, lw, aw);
-    p.out[(static_cast<int64_t>(b) * p.query_heads + g * G + h) * D + d] = lw > 0.0f ? aw / lw : 0.0f;
+    if constexpr (SPLIT) store_record(split_record(p, b, g, z, G, h, D), d, mx, lw, aw);
+    else p.out[(static_cast<int64_t>(b) * p.query_heads + g * G + h) * D + d] = lw > 0.0f ? aw / lw : 0.0f;
   }
-  if (APPEND && tid == 0) commit_sequence(p, b, len, n, commit);
+  if constexpr (SPLIT) finish_split<G, APPEND>(p, b, g, D, len, n, commit, &s_old);
+  else if (APPEND && tid == 0) commit_sequence(p, b, len, n, commit);
 }
 
 // (the online seal's builder state takes more registers: 2 resident
 // workgroups per compute unit, the fused grid's usual count, without spills)
 template <int G, int GR, bool APPEND, bool F16, bool ONLINE = false>
 __global__ __launch_bounds__(kThreads, ONLINE ? 2 : 4) void decode_kernel(const Params p) {
-  decode_body<G, GR, APPEND, F16, ONLINE>(p, NoProducer{});
+  decode_body<G, GR, APPEND, F16, ONLINE, false>(p, NoProducer{});
+}
+
+template <int G, int GR, bool APPEND, bool F16>
+__global__ __launch_bounds__(kThreads, 4) void decode_kernel_split(const Params p) {
+  decode_body<G, GR, APPEND, F16, false, true>(p, NoProducer{});
 }
 
 // The decode step fed by the q/k/v projection's partials (fp32 token).
 template <int G, int GR>
 __global__ __launch_bounds__(kThreads, 4) void decode_kernel_qkv(const Params p, const qkv::ReduceParams qp) {
-  decode_body<G, GR, true, false, false>(p, qp);
+  decode_body<G, GR, true, false, false, false>(p, qp);
 }
 
 // ---- shared selection: one block set per sequence over every query head -----
@@ -604,10 +770,11 @@ __device__ inline bool append_seal_shared(const Params& p, int b, int g, int64_t
 // G = query heads per KV head (1, 2 or 4; representatives per KV head, G
 // heads per representative row; the pages walked in registers); APPEND:
 // decode step; F16: raw FP16 K/V input.
-template <int G, bool APPEND, bool F16>
+template <int G, bool APPEND, bool F16, bool SPLIT>
 __global__ __launch_bounds__(kThreads) void decode_kernel_shared(const Params p) {
   const int g = blockIdx.x;
   const int b = blockIdx.y;
+  const int z = SPLIT ? blockIdx.z : 0;
   const int tid = threadIdx.x;
   const int wave = tid / kWave;
   const int lane = tid % kWave;
@@ -621,6 +788,7 @@ __global__ __launch_bounds__(kThreads) void decode_kernel_shared(const Params p)
   __shared__ uint32_t hist[256];
   __shared__ attn::CombineSmem<G, kWaves> cs;
   __shared__ ClaimSmem cl;
+  __shared__ uint32_t s_old;  // (SPLIT)
 
   const float* q_group = p.query + (static_cast<int64_t>(b) * p.query_heads + g * G) * D;
   int64_t len = p.seq_len[b];
@@ -630,7 +798,7 @@ __global__ __launch_bounds__(kThreads) void decode_kernel_shared(const Params p)
   if (APPEND) {
     commit.gen = p.generation ? p.generation[b] : 0;
     commit.appended = append_seal_shared<F16>(p, b, g, len, n, commit.added);
-    if (tid == 0) commit.arrived = atomicAdd(&p.arrive[b], 1);
+    if (!SPLIT && tid == 0) commit.arrived = atomicAdd(&p.arrive[b], 1);
   }
 
   attn::WaveState<G> st;
@@ -706,17 +874,18 @@ __global__ __launch_bounds__(kThreads) void decode_kernel_shared(const Params p)
     if (!n_ok || bs.bad) {
       if (lane == 0) {
         flag_status(p.v.status, n_ok ? kStatusBadBudget : kStatusCapacity);
-        if (g == 0) p.counts[b] = 0;
+        if (g == 0 && z == 0) p.counts[b] = 0;
       }
     } else {
-      count = sel::select_ids_wave(keys, n, bs, hist, g == 0 ? p.selected + static_cast<int64_t>(b) * p.sel_stride
-                                                              : nullptr,
+      const bool writes = g == 0 && z == 0;
+      count = sel::select_ids_wave(keys, n, bs, hist,
+                                   writes ? p.selected + static_cast<int64_t>(b) * p.sel_stride : nullptr,
                                    p.sel_stride, late);
-      if (lane == 0 && g == 0) p.counts[b] = count;
+      if (lane == 0 && writes) p.counts[b] = count;
     }
     list_late(p, b, cl, late, kKeys, count, fb, wn, tail_pages, lane);
   }
-  PlanPages src(cl, late, p.v, b, wave, fb.F, wn, wlen);
+  PlanPages<SPLIT> src(cl, late, p.v, b, wave, fb.F, wn, wlen, z, p.splits);
   for (;;) {
     const attn::PageRef pr = src.next(true);
     if (pr.valid <= 0) break;
@@ -731,9 +900,11 @@ __global__ __launch_bounds__(kThreads) void decode_kernel_shared(const Params p)
     const int d = o % D;
     float mx, lw, aw;
     attn::combine_element<G, kWaves>(cs, h, d, mx, lw, aw);
-    p.out[(static_cast<int64_t>(b) * p.query_heads + g * G + h) * D + d] = lw > 0.0f ? aw / lw : 0.0f;
+    if constexpr (SPLIT) store_record(split_record(p, b, g, z, G, h, D), d, mx, lw, aw);
+    else p.out[(static_cast<int64_t>(b) * p.query_heads + g * G + h) * D + d] = lw > 0.0f ? aw / lw : 0.0f;
   }
-  if (APPEND && tid == 0) commit_sequence(p, b, len, n, commit);
+  if constexpr (SPLIT) finish_split<G, APPEND>(p, b, g, D, len, n, commit, &s_old);
+  else if (APPEND && tid == 0) commit_sequence(p, b, len, n, commit);
 }
 
 
@@ -829,12 +1000,13 @@ __device__ inline float score_block_any(const Params& p, const float* q_s, int b
   return score;
 }
 
-template <int G, int LPR, bool F16>
+template <int G, int LPR, bool F16, bool SPLIT>
 __global__ __launch_bounds__(kThreads) void decode_kernel_rows(const Params p, int hd) {
   static_assert(G <= kRowsMaxG, "1, 2 or 4 query heads per KV head");
   using State = rows::RowsState<G, LPR>;
   const int g = blockIdx.x;
   const int b = blockIdx.y;
+  const int z = SPLIT ? blockIdx.z : 0;
   const int tid = threadIdx.x;
   const int wave = tid / kWave;
   const int lane = tid % kWave;
@@ -845,6 +1017,7 @@ __global__ __launch_bounds__(kThreads) void decode_kernel_rows(const Params p, i
   __shared__ ClaimSmem cl;
   __shared__ float w_ml[kWaves][G][2];
   __shared__ float w_acc[kWaves][G][LPR * 8];
+  __shared__ uint32_t s_old;  // (SPLIT)
 
   const int64_t out_row = static_cast<int64_t>(b) * p.v.kv_heads + g;
   const float* q_group = p.query + (static_cast<int64_t>(b) * p.query_heads + g * G) * hd;
@@ -855,7 +1028,7 @@ __global__ __launch_bounds__(kThreads) void decode_kernel_rows(const Params p, i
   SeqCommit commit{};
   commit.gen = p.generation ? p.generation[b] : 0;
   commit.appended = append_seal_head_any<F16>(p, b, g, hd, len, n, commit.added);
-  if (tid == 0) commit.arrived = atomicAdd(&p.arrive[b], 1);
+  if (!SPLIT && tid == 0) commit.arrived = atomicAdd(&p.arrive[b], 1);
 
   State st;
   st.init(q_group, hd, p.qscale, lane);
@@ -891,17 +1064,18 @@ __global__ __launch_bounds__(kThreads) void decode_kernel_rows(const Params p, i
     if (!n_ok || bs.bad) {
       if (lane == 0) {
         flag_status(p.v.status, n_ok ? kStatusBadBudget : kStatusCapacity);
-        p.counts[out_row] = 0;
+        if (z == 0) p.counts[out_row] = 0;
       }
     } else {
-      count = sel::select_ids_wave(keys, n, bs, hist, p.selected + out_row * p.sel_stride, p.sel_stride, late);
-      if (lane == 0) p.counts[out_row] = count;
+      count = sel::select_ids_wave(keys, n, bs, hist, z == 0 ? p.selected + out_row * p.sel_stride : nullptr,
+                                   p.sel_stride, late);
+      if (lane == 0 && z == 0) p.counts[out_row] = count;
     }
     list_late(p, b, cl, late, kMaxSelectBlocks, count, fb, wn, tail_pages, lane);
   }
   const int64_t lane_off = st.lane_offset(p.v.token_elems, g, hd);
   const int64_t v_off = static_cast<int64_t>(p.v.kv_heads) * hd;
-  PlanPages src(cl, late, p.v, b, wave, fb.F, wn, wlen);
+  PlanPages<SPLIT> src(cl, late, p.v, b, wave, fb.F, wn, wlen, z, p.splits);
   for (;;) {
     const attn::PageRef pr = src.next(true);
     if (pr.valid <= 0) break;
@@ -936,9 +1110,11 @@ __global__ __launch_bounds__(kThreads) void decode_kernel_rows(const Params p, i
         aw += w_acc[w][h][d] * f;
       }
     }
-    p.out[(static_cast<int64_t>(b) * p.query_heads + g * G + h) * hd + d] = lw > 0.0f ? aw / lw : 0.0f;
+    if constexpr (SPLIT) store_record(split_record(p, b, g, z, G, h, hd), d, mx, lw, aw);
+    else p.out[(static_cast<int64_t>(b) * p.query_heads + g * G + h) * hd + d] = lw > 0.0f ? aw / lw : 0.0f;
   }
-  if (tid == 0) commit_sequence(p, b, len, n, commit);
+  if constexpr (SPLIT) finish_split<G, true>(p, b, g, hd, len, n, commit, &s_old);
+  else if (tid == 0) commit_sequence(p, b, len, n, commit);
 }
 
 
@@ -951,17 +1127,21 @@ __global__ __launch_bounds__(kThreads) void decode_kernel_rows(const Params p, i
 // on v_mfma_f32_16x16x32_f16), one page in flight while the previous one is
 // computed.  A step that seals nothing stores its token at the start of the
 // walk phase (wave 0, before it lists the tail).
-template <int GR, bool APPEND, bool F16, bool ONLINE = false>
+template <int G, int GR, bool APPEND, bool F16, bool ONLINE = false, bool SPLIT = false>
 __global__ __launch_bounds__(kThreads) void decode_kernel_staged(const Params p) {
-  constexpr int G = 4;
+  static_assert(G == 4 || G == 8, "the staged walk");
+  static_assert(!SPLIT || !ONLINE, "the workgroups of a list would all run its online seal");
+  // the waves' states meet row by row where that fits the page slots
+  constexpr bool kCombineRows = sizeof(attn::CombineRowsSmem<G, kWaves>) <= kWaves * attn::kStageVecs * 16;
   constexpr int kStageBytes = kWaves * attn::kStageVecs * 16;
   constexpr int kPbufFloats = (G * 32 + G + 3) / 4 * 4;
   constexpr int kSlotBytes = attn::kStageVecs * 16;
   static_assert(kMaxSelectBlocks * 4 <= 2 * kSlotBytes, "keys fit the page slots of waves 0 and 1");
-  static_assert(sizeof(attn::CombineRowsSmem<G, kWaves>) <= kStageBytes, "combine fits the page slots");
+  static_assert(sizeof(attn::CombineSmem<G, kWaves>) <= kStageBytes, "combine fits the page slots");
   static_assert(kEarly <= kWave, "one lane per early lookup");
   const int g = blockIdx.x;
   const int b = blockIdx.y;
+  const int z = SPLIT ? blockIdx.z : 0;
   const int tid = threadIdx.x;
   const int wave = tid / kWave;
   const int lane = tid % kWave;
@@ -976,6 +1156,7 @@ __global__ __launch_bounds__(kThreads) void decode_kernel_staged(const Params p)
   __shared__ uint32_t hist[256];
   __shared__ ClaimSmem cl;
   __shared__ int32_t late_ids[kStagedIds + kTailPages];  // the selected ids, then (in place) the late pages
+  __shared__ uint32_t s_old;  // (SPLIT)
   uint32_t* keys = reinterpret_cast<uint32_t*>(smem);
   uint4* stage = reinterpret_cast<uint4*>(smem) + wave * attn::kStageVecs;
   float* pbuf = pbuf_s + wave * kPbufFloats;
@@ -983,7 +1164,10 @@ __global__ __launch_bounds__(kThreads) void decode_kernel_staged(const Params p)
 
   const int64_t out_row = static_cast<int64_t>(b) * p.v.kv_heads + g;
   // the group's query rows, loaded at entry (their latency overlaps the append)
-  const float q_entry = q_group[tid % (G * D)];
+  constexpr int kQLoads = G * D / kThreads;
+  float q_entry[kQLoads];
+#pragma unroll
+  for (int i = 0; i < kQLoads; ++i) q_entry[i] = q_group[i * kThreads + tid];
   int64_t len = p.seq_len[b];
   int n = p.sealed[b];
 
@@ -1007,7 +1191,7 @@ __global__ __launch_bounds__(kThreads) void decode_kernel_staged(const Params p)
       tail_page = table_page(p.v, b, len / kPageTokens);
       if (wave == 0) token = token_quad<F16>(p, b, g, lane);
     }
-    if (tid == 0) commit.arrived = atomicAdd(&p.arrive[b], 1);
+    if (!SPLIT && tid == 0) commit.arrived = atomicAdd(&p.arrive[b], 1);
   }
 
   attn::WaveState<G> st;
@@ -1032,17 +1216,21 @@ __global__ __launch_bounds__(kThreads) void decode_kernel_staged(const Params p)
     a.group = G;
     a.rep_heads = p.rep_heads;
     a.rep_stride = p.rep_stride;
-    static_assert(G * D == kThreads, "one query element per thread");
-    q_t[(tid % D) * G + tid / D] = q_entry;
+    static_assert(G * D % kThreads == 0 && kThreads % D == 0, "whole query rows per pass of the workgroup");
+#pragma unroll
+    for (int i = 0; i < kQLoads; ++i) q_t[(tid % D) * G + tid / D + i * (kThreads / D)] = q_entry[i];
     __syncthreads();
     sel::score_blocks_vec<GR, 2, kThreads>(a, q_t, n, keys, nullptr, tid);
   }
   if (ONLINE && deferred && tail_page >= 0) {
     // the group's query rows of this step to the ring (read by later seals)
     const int64_t slot = len % p.online.ring_tokens;
-    const int h = g * G + tid / D;
-    p.online.ring[((static_cast<int64_t>(b) * p.online.query_heads + h) * p.online.ring_tokens + slot) * D +
-                  tid % D] = q_entry;
+#pragma unroll
+    for (int i = 0; i < kQLoads; ++i) {
+      const int h = g * G + tid / D + i * (kThreads / D);
+      p.online.ring[((static_cast<int64_t>(b) * p.online.query_heads + h) * p.online.ring_tokens + slot) * D +
+                    tid % D] = q_entry[i];
+    }
   }
   if (wave == kWaves - 1) cl.early[lane] = early;
   if (tid == 0) cl.late_ready = 0;
@@ -1073,31 +1261,41 @@ __global__ __launch_bounds__(kThreads) void decode_kernel_staged(const Params p)
     if (!n_ok || bs.bad) {
       if (lane == 0) {
         flag_status(p.v.status, n_ok ? kStatusBadBudget : kStatusCapacity);
-        p.counts[out_row] = 0;
+        if (z == 0) p.counts[out_row] = 0;
       }
     } else {
-      count = sel::select_ids_wave(keys, n, bs, hist, p.selected + out_row * p.sel_stride, p.sel_stride, late_ids);
-      if (lane == 0) p.counts[out_row] = count;
+      count = sel::select_ids_wave(keys, n, bs, hist, z == 0 ? p.selected + out_row * p.sel_stride : nullptr,
+                                   p.sel_stride, late_ids);
+      if (lane == 0 && z == 0) p.counts[out_row] = count;
     }
     list_late(p, b, cl, late_ids, kStagedIds + kTailPages, count, fb, wn, tail_pages, lane);
   }
   const bool waits = wave != 0 && wave * kSlotBytes < n * 4;  // the keys reach into this wave's page slot
   if (waits) wait_late(cl);
-  PlanPages src(cl, late_ids, p.v, b, wave, fb.F, wn, wlen);
+  PlanPages<SPLIT> src(cl, late_ids, p.v, b, wave, fb.F, wn, wlen, z, p.splits);
   st.attend_staged(p.v, src, lg, lane, g, stage, pbuf, q_group, p.qscale);
   __syncthreads();  // every wave is done with its slot before the combine reuses the area
 
-  attn::CombineRowsSmem<G, kWaves>& cs = *reinterpret_cast<attn::CombineRowsSmem<G, kWaves>*>(smem);
-  attn::publish_wave_rows<G, kWaves>(st, cs, wave, lg.row, lg.col);
+  using Combine = std::conditional_t<kCombineRows, attn::CombineRowsSmem<G, kWaves>, attn::CombineSmem<G, kWaves>>;
+  Combine& cs = *reinterpret_cast<Combine*>(smem);
+  if constexpr (kCombineRows) {
+    attn::publish_wave_rows<G, kWaves>(st, cs, wave, lg.row, lg.col);
+  } else {
+    st.reduce_rows();
+    attn::publish_wave<G, kWaves>(st, cs, wave, lane, lg.row, lg.col);
+  }
   __syncthreads();
   for (int o = tid; o < G * D; o += kThreads) {
     const int h = o / D;
     const int d = o % D;
     float mx, lw, aw;
-    attn::combine_element_rows<G, kWaves>(cs, h, d, mx, lw, aw);
-    p.out[(static_cast<int64_t>(b) * p.query_heads + g * G + h) * D + d] = lw > 0.0f ? aw / lw : 0.0f;
+    if constexpr (kCombineRows) attn::combine_element_rows<G, kWaves>(cs, h, d, mx, lw, aw);
+    else attn::combine_element<G, kWaves>(cs, h, d, mx, lw, aw);
+    if constexpr (SPLIT) store_record(split_record(p, b, g, z, G, h, D), d, mx, lw, aw);
+    else p.out[(static_cast<int64_t>(b) * p.query_heads + g * G + h) * D + d] = lw > 0.0f ? aw / lw : 0.0f;
   }
-  if (APPEND && tid == 0) commit_sequence(p, b, len, n, commit);
+  if constexpr (SPLIT) finish_split<G, APPEND>(p, b, g, D, len, n, commit, &s_old);
+  else if (APPEND && tid == 0) commit_sequence(p, b, len, n, commit);
 }
 
 // Decode step with the InfLLM online seal (fp32 K/V, one representative per
@@ -1107,7 +1305,7 @@ hipError_t launch_online(const Params& p, int batch, hipStream_t stream) {
   const dim3 grid(p.v.kv_heads, batch);
   if (p.rep_heads != p.query_heads) return hipErrorInvalidValue;
   if (group == 4) {
-    hipLaunchKernelGGL((decode_kernel_staged<1, true, false, true>), grid, dim3(kThreads), 0, stream, p);
+    hipLaunchKernelGGL((decode_kernel_staged<4, 1, true, false, true>), grid, dim3(kThreads), 0, stream, p);
   } else if (group == 1) {
     hipLaunchKernelGGL((decode_kernel<1, 1, true, false, true>), grid, dim3(kThreads), 0, stream, p);
   } else {
@@ -1123,9 +1321,9 @@ hipError_t launch_mode(const Params& p, int batch, hipStream_t stream) {
   const dim3 grid(p.v.kv_heads, batch);
   if (group == 4) {
     if (per_query_reps) {
-      hipLaunchKernelGGL((decode_kernel_staged<1, APPEND, F16>), grid, dim3(kThreads), 0, stream, p);
+      hipLaunchKernelGGL((decode_kernel_staged<4, 1, APPEND, F16>), grid, dim3(kThreads), 0, stream, p);
     } else {
-      hipLaunchKernelGGL((decode_kernel_staged<4, APPEND, F16>), grid, dim3(kThreads), 0, stream, p);
+      hipLaunchKernelGGL((decode_kernel_staged<4, 4, APPEND, F16>), grid, dim3(kThreads), 0, stream, p);
     }
   } else if (group == 1) {
     hipLaunchKernelGGL((decode_kernel<1, 1, APPEND, F16>), grid, dim3(kThreads), 0, stream, p);
@@ -1167,16 +1365,88 @@ bool select_attend_shared_supported(int32_t batch, int32_t query_heads, int32_t 
   return repeat <= kSharedRepeatBytes;
 }
 
-template <bool APPEND, bool F16>
+template <bool APPEND, bool F16, bool SPLIT = false>
 hipError_t launch_shared(const Params& p, int batch, hipStream_t stream) {
-  const dim3 grid(p.v.kv_heads, batch);
+  const dim3 grid(p.v.kv_heads, batch, SPLIT ? p.splits : 1);
   const int group = p.query_heads / p.v.kv_heads;
   if (group == 1) {
-    hipLaunchKernelGGL((decode_kernel_shared<1, APPEND, F16>), grid, dim3(kThreads), 0, stream, p);
+    hipLaunchKernelGGL((decode_kernel_shared<1, APPEND, F16, SPLIT>), grid, dim3(kThreads), 0, stream, p);
   } else if (group == 2) {
-    hipLaunchKernelGGL((decode_kernel_shared<2, APPEND, F16>), grid, dim3(kThreads), 0, stream, p);
+    hipLaunchKernelGGL((decode_kernel_shared<2, APPEND, F16, SPLIT>), grid, dim3(kThreads), 0, stream, p);
   } else {
-    hipLaunchKernelGGL((decode_kernel_shared<4, APPEND, F16>), grid, dim3(kThreads), 0, stream, p);
+    hipLaunchKernelGGL((decode_kernel_shared<4, APPEND, F16, SPLIT>), grid, dim3(kThreads), 0, stream, p);
+  }
+  return hipGetLastError();
+}
+
+// ---- the step with several workgroups per list ----------------------------------
+// Every workgroup of a list scores all of it, so long lists are left to the
+// launches that share the scores.
+constexpr int kMaxSplitStepBlocks = 1024;
+
+// Bits of a KV head's field in a sequence's 32-bit arrival counter.
+static int split_field_bits(int32_t kv_heads) {
+  const int bits = kv_heads > 0 ? 32 / kv_heads : 0;
+  return bits > 8 ? 8 : bits;
+}
+
+int32_t split_step_cap(int32_t batch, int32_t query_heads, int32_t kv_heads, int32_t head_dim) {
+  if (batch <= 0 || kv_heads <= 0) return 1;
+  const int bits = split_field_bits(kv_heads);
+  if (bits < 1) return 1;
+  const int64_t lists = static_cast<int64_t>(batch) * kv_heads;
+  const int64_t slots =
+      (head_dim == kHeadDim && query_heads / kv_heads >= 4 ? 1 : 2) * static_cast<int64_t>(compute_units());
+  const int64_t most = (int64_t{1} << bits) - 1 < kMaxStepSplits ? (int64_t{1} << bits) - 1 : kMaxStepSplits;
+  const int64_t want = slots / lists;
+  return static_cast<int32_t>(want < 1 ? 1 : (want < most ? want : most));
+}
+
+int32_t split_step_splits(const SelectAttendLaunch& s) {
+  if (s.ring || s.kv_heads <= 0 || s.rep_stride > kMaxSplitStepBlocks || split_field_bits(s.kv_heads) < 1) return 0;
+  const int hd = s.head_dim > 0 ? s.head_dim : kHeadDim;
+  const int group = s.query_heads / s.kv_heads;
+  const bool shared = s.select_groups != s.kv_heads;
+  if (hd != kHeadDim) {
+    if (!s.append || !select_attend_rows_supported(s.query_heads, s.kv_heads, s.rep_heads, s.select_groups, hd))
+      return 0;
+  } else if (shared) {
+    if (!select_attend_shared_supported(s.batch, s.query_heads, s.kv_heads, s.rep_heads, s.select_groups,
+                                        s.rep_stride))
+      return 0;
+  } else if (group == 8) {
+    if (s.sel_stride > kStagedIds || !sel::vec_layout<2>(s.reps, s.rep_stride)) return 0;
+  } else if (!select_attend_supported(s.query_heads, s.kv_heads, s.select_groups, s.sel_stride, s.reps,
+                                      s.rep_stride)) {
+    return 0;
+  }
+  const int32_t cap = split_step_cap(s.batch, s.query_heads, s.kv_heads, hd);
+  const int32_t pages = s.budget + 1;  // (a partial tail page)
+  const int32_t by_pages = pages / kWaves < 1 ? 1 : pages / kWaves;
+  return cap < by_pages ? cap : by_pages;
+}
+
+template <bool APPEND, bool F16>
+hipError_t launch_split(const Params& p, int batch, hipStream_t stream) {
+  const int group = p.query_heads / p.v.kv_heads;
+  const bool per_query_reps = p.rep_heads == p.query_heads;
+  const dim3 grid(p.v.kv_heads, batch, p.splits), block(kThreads);
+  if (group == 8) {
+    if (per_query_reps)
+      hipLaunchKernelGGL((decode_kernel_staged<8, 1, APPEND, F16, false, true>), grid, block, 0, stream, p);
+    else
+      hipLaunchKernelGGL((decode_kernel_staged<8, 8, APPEND, F16, false, true>), grid, block, 0, stream, p);
+  } else if (group == 4) {
+    if (per_query_reps)
+      hipLaunchKernelGGL((decode_kernel_staged<4, 1, APPEND, F16, false, true>), grid, block, 0, stream, p);
+    else
+      hipLaunchKernelGGL((decode_kernel_staged<4, 4, APPEND, F16, false, true>), grid, block, 0, stream, p);
+  } else if (group == 1) {
+    hipLaunchKernelGGL((decode_kernel_split<1, 1, APPEND, F16>), grid, block, 0, stream, p);
+  } else if (per_query_reps) {
+    hipLaunchKernelGGL((decode_kernel_split<2, 1, APPEND, F16>), grid, block, 0, stream, p);
+  } else {
+    hipLaunchKernelGGL((decode_kernel_split<2, 2, APPEND, F16>), grid, block, 0, stream, p);
   }
   return hipGetLastError();
 }
@@ -1189,23 +1459,23 @@ bool select_attend_rows_supported(int32_t query_heads, int32_t kv_heads, int32_t
          head_dim <= rows::kMaxHeadDim && head_dim != kHeadDim;
 }
 
-template <int LPR, bool F16>
+template <int LPR, bool F16, bool SPLIT>
 hipError_t launch_rows_step(const Params& p, int batch, int hd, hipStream_t stream) {
-  const dim3 grid(p.v.kv_heads, batch);
+  const dim3 grid(p.v.kv_heads, batch, SPLIT ? p.splits : 1), block(kThreads);
   switch (p.query_heads / p.v.kv_heads) {
-    case 1: hipLaunchKernelGGL((decode_kernel_rows<1, LPR, F16>), grid, dim3(kThreads), 0, stream, p, hd); break;
-    case 2: hipLaunchKernelGGL((decode_kernel_rows<2, LPR, F16>), grid, dim3(kThreads), 0, stream, p, hd); break;
-    default: hipLaunchKernelGGL((decode_kernel_rows<4, LPR, F16>), grid, dim3(kThreads), 0, stream, p, hd); break;
+    case 1: hipLaunchKernelGGL((decode_kernel_rows<1, LPR, F16, SPLIT>), grid, block, 0, stream, p, hd); break;
+    case 2: hipLaunchKernelGGL((decode_kernel_rows<2, LPR, F16, SPLIT>), grid, block, 0, stream, p, hd); break;
+    default: hipLaunchKernelGGL((decode_kernel_rows<4, LPR, F16, SPLIT>), grid, block, 0, stream, p, hd); break;
   }
   return hipGetLastError();
 }
 
-template <bool F16>
+template <bool F16, bool SPLIT = false>
 hipError_t launch_rows_lpr(const Params& p, int batch, int hd, hipStream_t stream) {
   switch (rows::lanes_per_row(hd)) {
-    case 8: return launch_rows_step<8, F16>(p, batch, hd, stream);
-    case 16: return launch_rows_step<16, F16>(p, batch, hd, stream);
-    default: return launch_rows_step<32, F16>(p, batch, hd, stream);
+    case 8: return launch_rows_step<8, F16, SPLIT>(p, batch, hd, stream);
+    case 16: return launch_rows_step<16, F16, SPLIT>(p, batch, hd, stream);
+    default: return launch_rows_step<32, F16, SPLIT>(p, batch, hd, stream);
   }
 }
 
@@ -1280,6 +1550,25 @@ hipError_t launch_select_attend(const SelectAttendLaunch& s, hipStream_t stream)
   }
   if (!s.append) return launch_mode<false, false>(p, s.batch, stream);
   return s.k16 ? launch_mode<true, true>(p, s.batch, stream) : launch_mode<true, false>(p, s.batch, stream);
+}
+
+hipError_t launch_split_step(const SelectAttendLaunch& s, float* records, int32_t splits, hipStream_t stream) {
+  const int hd = s.head_dim > 0 ? s.head_dim : kHeadDim;
+  if (!s.arrive || !records || splits < 1 || splits > split_step_splits(s)) return hipErrorInvalidValue;
+  Params p = step_params(s, hd);
+  p.part = records;
+  p.splits = splits;
+  p.field_bits = split_field_bits(s.kv_heads);
+  if (hd != kHeadDim)
+    return s.k16 ? launch_rows_lpr<true, true>(p, s.batch, hd, stream)
+                 : launch_rows_lpr<false, true>(p, s.batch, hd, stream);
+  if (s.select_groups != s.kv_heads) {
+    if (!s.append) return launch_shared<false, false, true>(p, s.batch, stream);
+    return s.k16 ? launch_shared<true, true, true>(p, s.batch, stream)
+                 : launch_shared<true, false, true>(p, s.batch, stream);
+  }
+  if (!s.append) return launch_split<false, false>(p, s.batch, stream);
+  return s.k16 ? launch_split<true, true>(p, s.batch, stream) : launch_split<true, false>(p, s.batch, stream);
 }
 
 bool decode_step_qkv_supported(int32_t query_heads, int32_t kv_heads, int32_t select_groups, int32_t head_dim) {
