@@ -326,8 +326,7 @@ struct WaveState {
         if ((it0 + it * it_step) * kRows + row >= valid) s[h][it] = kNegInf;
         pmax = fmaxf(pmax, s[h][it]);
       }
-      pmax = fmaxf(pmax, shfl_xor_f(pmax, 16));
-      pmax = fmaxf(pmax, shfl_xor_f(pmax, 32));
+      pmax = xor_max<32>(xor_max<16>(pmax));
       const float mn = fmaxf(m[h], pmax);
       // mn == -inf only if nothing finite was seen: the state stays empty
       const float corr = (m[h] == mn) ? 1.0f : __builtin_amdgcn_exp2f(m[h] - mn);
@@ -440,8 +439,7 @@ struct WaveState {
           amax = fmaxf(amax, fabsf(x[kk][j]));
         }
       }
-      amax = fmaxf(amax, shfl_xor_f(amax, 16));
-      amax = fmaxf(amax, shfl_xor_f(amax, 32));
+      amax = xor_max<32>(xor_max<16>(amax));
       const int ex = static_cast<int>((__float_as_uint(amax) >> 23) & 0xff);
       const int sh = ex == 0 ? 0 : min(126, max(-126, 140 - ex));  // amax * 2^sh in [2^13, 2^14)
       const float scale = __uint_as_float(static_cast<uint32_t>(127 + sh) << 23);
@@ -518,8 +516,7 @@ struct WaveState {
       float pmax = kNegInf;
 #pragma unroll
       for (int e = 0; e < 8; ++e) pmax = fmaxf(pmax, sv[e]);
-      pmax = fmaxf(pmax, shfl_xor_f(pmax, 16));
-      pmax = fmaxf(pmax, shfl_xor_f(pmax, 32));
+      pmax = xor_max<32>(xor_max<16>(pmax));
       const float mn = fmaxf(m_lane, pmax);
       const float corr = (m_lane == mn) ? 1.0f : __builtin_amdgcn_exp2f(m_lane - mn);
       const float base_m = (mn == kNegInf) ? 0.0f : mn;
@@ -598,13 +595,9 @@ struct WaveState {
   __device__ inline void reduce_rows() {
 #pragma unroll
     for (int h = 0; h < G; ++h) {
-      l[h] += shfl_xor_f(l[h], 16);
-      l[h] += shfl_xor_f(l[h], 32);
+      l[h] = xor_sum<32>(xor_sum<16>(l[h]));
 #pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        acc[h][j] += shfl_xor_f(acc[h][j], 16);
-        acc[h][j] += shfl_xor_f(acc[h][j], 32);
-      }
+      for (int j = 0; j < 8; ++j) acc[h][j] = xor_sum<32>(xor_sum<16>(acc[h][j]));
     }
   }
 };

@@ -43,23 +43,23 @@ __device__ inline float lane_row_sum(float v) {
   } else {
     static_assert(LPR == 32, "8, 16 or 32 lanes per row");
     v = row16_sum(v);
-    return v + shfl_xor_f(v, 16);
+    return xor_sum<16>(v);
   }
 }
 
 // Sum / max over the token rows of a wave (the lanes of one column).
 template <int LPR>
 __device__ inline float across_rows_sum(float v) {
-#pragma unroll
-  for (int o = LPR; o < kWave; o <<= 1) v += shfl_xor_f(v, o);
-  return v;
+  if constexpr (LPR <= 8) v = xor_sum<8>(v);
+  if constexpr (LPR <= 16) v = xor_sum<16>(v);
+  return xor_sum<32>(v);
 }
 
 template <int LPR>
 __device__ inline float across_rows_max(float v) {
-#pragma unroll
-  for (int o = LPR; o < kWave; o <<= 1) v = fmaxf(v, shfl_xor_f(v, o));
-  return v;
+  if constexpr (LPR <= 8) v = xor_max<8>(v);
+  if constexpr (LPR <= 16) v = xor_max<16>(v);
+  return xor_max<32>(v);
 }
 
 // Online-softmax state of one wave for the G query heads of a KV head.

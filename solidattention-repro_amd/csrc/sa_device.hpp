@@ -139,8 +139,42 @@ __device__ inline uint32_t wave_prefix_sum(uint32_t v) {
   return v;
 }
 
-__device__ inline float shfl_xor_f(float v, int mask) {
-  return __shfl_xor(v, mask, kWave);
+// Sum / max with the lane 8, 16 or 32 lanes away, on the VALU: a rotation by 8
+// within a 16-lane row, and the row and half exchanges of gfx950
+// (v_permlane16_swap: odd rows of one register against even rows of the
+// other; v_permlane32_swap: the halves), each of which leaves both partners'
+// values in a pair of registers.  __shfl_xor goes through the LDS pipe: at 8
+// query heads per KV head the waves' closing row sums alone, 144 exchanges
+// each, took 4 of 5 us.
+struct LanePair {
+  float a;
+  float b;
+};
+__device__ inline LanePair pair_xor16(float v) {
+  const uint32_t u = __builtin_bit_cast(uint32_t, v);
+  const auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+  return LanePair{__builtin_bit_cast(float, static_cast<uint32_t>(r[0])), __builtin_bit_cast(float, static_cast<uint32_t>(r[1]))};
+}
+__device__ inline LanePair pair_xor32(float v) {
+  const uint32_t u = __builtin_bit_cast(uint32_t, v);
+  const auto r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+  return LanePair{__builtin_bit_cast(float, static_cast<uint32_t>(r[0])), __builtin_bit_cast(float, static_cast<uint32_t>(r[1]))};
+}
+constexpr int kDppRowRor8 = 0x128;  // row_ror:8, lane ^ 8
+
+template <int Mask>
+__device__ inline float xor_sum(float v) {
+  static_assert(Mask == 8 || Mask == 16 || Mask == 32, "rotation, row or half exchange");
+  if constexpr (Mask == 8) return v + dpp_f<kDppRowRor8>(v);
+  const LanePair p = Mask == 16 ? pair_xor16(v) : pair_xor32(v);
+  return p.a + p.b;
+}
+template <int Mask>
+__device__ inline float xor_max(float v) {
+  static_assert(Mask == 8 || Mask == 16 || Mask == 32, "rotation, row or half exchange");
+  if constexpr (Mask == 8) return fmaxf(v, dpp_f<kDppRowRor8>(v));
+  const LanePair p = Mask == 16 ? pair_xor16(v) : pair_xor32(v);
+  return fmaxf(p.a, p.b);
 }
 
 // ---- synthetic data (bit-identical to the host generator) ----------------

@@ -207,9 +207,9 @@ __device__ inline void commit_sequence(const Params& p, int b, int64_t len, int 
 // wave) rather than bytes, and before by launches: append + seal, scoring,
 // selection, attention and merge cost about 4.5 us each even with nothing to
 // do.  Per layer, as those launches and as this one: 16 sequences of 4-8K
-// tokens, 16/8 heads 51 -> 35 us; 16 x 8-16K, 64/8 heads 62 -> 54 us; 32 x
+// tokens, 16/8 heads 51 -> 35 us; 16 x 8-16K, 64/8 heads 62 -> 51 us; 32 x
 // 5-10K, 16/8 heads of 64: 59 -> 42 us; 4 x 4-8K with online
-// representatives (append + seal in its own launch) 54 -> 38 us.
+// representatives (append + seal in its own launch) 54 -> 35 us.
 struct SplitEnd {
   bool list_last;
   bool seq_last;
@@ -441,16 +441,21 @@ struct PlanPages {
   }
 
   // The split plan: walker u = wave * splits + z of 8 * splits (<= 128), the
-  // selecting waves first; the same balance as below, each lane planning two
-  // walkers and a prefix sum giving where a walker's range begins.
+  // selecting waves first.  No wave has a late position before its
+  // workgroup's selection is done, so a walker starts on them after the
+  // larger of its forced positions and the selection (kSelectPages), and the
+  // ranges even out the sums.  Each lane plans two walkers; a prefix sum gives
+  // where a walker's range begins.
   __device__ inline int split_want(int u, int late_n) const {
     const int walkers = kWaves * splits;
     if (u >= walkers) return 0;
-    const int total = F + late_n + kSelectPages * splits;
+    const int step = (kWaves - 1) * splits;
+    const int each = F / step, more = F % step;  // forced positions: each + 1 for the first `more` ranks
+    const int base = max(each, kSelectPages), base_more = max(each + 1, kSelectPages);
+    const int total = late_n + kSelectPages * splits + more * base_more + (step - more) * base;
     const int target = total / walkers + (u < total % walkers ? 1 : 0);
     const int r = u - splits;  // rank among the forced positions' walkers
-    const int step = (kWaves - 1) * splits;
-    const int want = target - (r < 0 ? kSelectPages : (r < F ? (F - r + step - 1) / step : 0));
+    const int want = target - (r < 0 ? kSelectPages : (r < more ? base_more : base));
     return want > 0 ? want : 0;
   }
   __device__ inline void plan_late_split(int late_n) {
@@ -530,6 +535,85 @@ struct PlanPages {
 // G = query heads per KV head; GR = query heads sharing one representative
 // row (G for per-KV-head representatives, 1 for per-query-head ones);
 // APPEND: decode step (append + seal first); F16: raw FP16 K/V input.
+// Scores with every lane of the workgroup loading, 256 blocks at a time: lanes
+// tid and tid + 256 share a block.  With one representative row (GR == G) each
+// takes 64 of its 128 values, all in flight at once, and the first lane's
+// partial dots are handed to the second, which goes on with the sum (while the
+// first loads the next 256 blocks); with a row per query head (G = 2) each
+// takes a row.  The reference's operations in its order, as sel::score_one().
+// part: 2 G * 256 floats of LDS.  One lane per block leaves half the waves
+// idle up to 256 blocks and takes two or more round trips to memory.
+template <int G, int GR>
+__device__ inline void score_halves(const sel::ScoreArgs& a, const float* q_s, int n, uint32_t* keys, float* part,
+                                    float (&pre)[sel::kScoreBatch], bool have_pre) {
+  constexpr int kHalf = kThreads / 2;
+  constexpr int kB = sel::kScoreBatch;
+  static_assert(D == 2 * kB, "two batches per representative row");
+  static_assert(GR == G || (G == 2 && GR == 1), "one row, or a half of the lanes per row");
+  const int half = threadIdx.x / kHalf;  // wave-uniform
+  const float heads_f = static_cast<float>(a.heads_per_sel);
+  int qoff = 0;
+  asm volatile("" : "+s"(qoff));
+  auto sum = [&](float (&dot)[GR], int h0, int d0) {
+#pragma unroll
+    for (int k = 0; k < kB; ++k) {
+      // the query reads in steps of 16 (all of them read ahead would spill)
+      if (k % 16 == 0) __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int j = 0; j < GR; ++j) dot[j] = dot[j] + q_s[qoff + (h0 + j) * D + d0 + k] * pre[k];
+    }
+  };
+  for (int c0 = 0; c0 < n; c0 += kHalf) {
+    const int slot = threadIdx.x % kHalf;
+    const int blk = c0 + slot;
+    const bool valid = blk < n;
+    sel::ScoreArgs row = a;
+    asm volatile("" : "+s"(row.rep_stride));  // (or 64 row offsets are kept across the iterations, and spill)
+    // alternating, so that one barrier per 256 blocks separates reads and writes
+    float* part_c = part + (c0 / kHalf % 2) * G * kHalf + slot;
+    if constexpr (GR == G) {
+      float dot[G];
+#pragma unroll
+      for (int j = 0; j < G; ++j) dot[j] = 0.0f;
+      if (valid && !(have_pre && c0 == 0)) sel::score_prefetch(row, blk, pre, half * kB);
+      if (half == 1) {
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < G; ++j) dot[j] = part_c[j * kHalf];
+      }
+      if (valid) sum(dot, 0, half * kB);
+      if (half == 0) {
+#pragma unroll
+        for (int j = 0; j < G; ++j) part_c[j * kHalf] = dot[j];
+        __syncthreads();
+      } else if (valid) {
+        float score = 0.0f;
+#pragma unroll
+        for (int j = 0; j < G; ++j) score = score + dot[j] / heads_f;
+        keys[blk] = sel::order_key(score);
+      }
+    } else {
+      if (valid) {
+        row.h_first = a.h_first + half;
+        float dot[1] = {0.0f};
+#pragma unroll
+        for (int d0 = 0; d0 < D; d0 += kB) {
+          sel::score_prefetch(row, blk, pre, d0);
+          sum(dot, half, d0);
+        }
+        part_c[half * kHalf] = dot[0];
+      }
+      __syncthreads();
+      if (valid && half == 0) {
+        float score = 0.0f;
+#pragma unroll
+        for (int j = 0; j < G; ++j) score = score + part_c[j * kHalf] / heads_f;
+        keys[blk] = sel::order_key(score);
+      }
+    }
+  }
+}
+
 // No q/k/v producer: the step's query and token are inputs.
 struct NoProducer {};
 
@@ -602,9 +686,13 @@ __device__ inline void decode_body(const Params& p, const Prod& qp) {
   // (with one representative row per query head the group's G rows would
   // keep the prefetched batch live across the second row: not prefetched)
   constexpr bool kPrefetch = GR == G;
-  const bool have_pre = kPrefetch && n >= 0 && n <= p.rep_stride && n <= kMaxSelectBlocks && tid < n;
+  // SPLIT: lanes tid and tid + 256 share a block (see score_halves()) and each
+  // prefetches its half
+  constexpr int kHalf = kThreads / 2;
+  const bool have_pre = kPrefetch && n >= 0 && n <= p.rep_stride &&
+                        n <= kMaxSelectBlocks && (SPLIT ? tid % kHalf : tid) < n;
   float pre[sel::kScoreBatch];
-  if (have_pre) sel::score_prefetch(a, tid, pre);
+  if (have_pre) sel::score_prefetch(a, SPLIT ? tid % kHalf : tid, pre, SPLIT ? tid / kHalf * sel::kScoreBatch : 0);
 
   // ---- 1. append + seal (decode step) ---------------------------------------
   // The arrival count is read at the end of the kernel, so that its round
@@ -631,7 +719,9 @@ __device__ inline void decode_body(const Params& p, const Prod& qp) {
   if (n_ok && !bs.take_all) {  // (a budget that takes every block needs no scores)
     if (!kProd && tid < G * D) q_s[tid] = q_entry;
     __syncthreads();
-    if (kPrefetch) {
+    if constexpr (SPLIT) {
+      score_halves<G, GR>(a, q_s, n, keys, reinterpret_cast<float*>(&cs), pre, have_pre);
+    } else if constexpr (kPrefetch) {
       sel::score_blocks<GR, kThreads>(a, q_s, n, keys, nullptr, pre, have_pre);
     } else {
       sel::score_blocks<GR, kThreads>(a, q_s, n, keys, nullptr);
@@ -835,7 +925,8 @@ __global__ __launch_bounds__(kThreads) void decode_kernel_shared(const Params p)
       if (blk < n) {
         for (int h0 = wave * G; h0 < hps; h0 += kWaves * G) {
           float dot[G][1];
-          sel::row_dots<G, 1, 32>(a, q_t, blk, h0, dot);
+          if constexpr (SPLIT) sel::row_dots_at_once<G>(a, q_t, blk, h0, dot);
+          else sel::row_dots<G, 1, 32>(a, q_t, blk, h0, dot);
 #pragma unroll
           for (int j = 0; j < G; ++j) dots[h0 + j][lane] = dot[j][0];
         }
@@ -975,7 +1066,8 @@ __device__ inline bool append_seal_head_any(const Params& p, int b, int g, int h
 // q_s = the G query rows of hd floats in LDS.
 template <int G>
 __device__ inline float score_block_any(const Params& p, const float* q_s, int b, int g, int hd, int blk) {
-  constexpr int kBatch = 32;
+  constexpr int kBatch = 64;  // (a whole row at head_dim 64: one round trip to memory)
+  constexpr int kStep = 8;    // head_dim is a multiple of 8
   const int64_t stride = p.rep_stride;
   const float* r = p.reps + (static_cast<int64_t>(b) * p.rep_heads + g) * hd * stride + blk;
   float dot[G];
@@ -984,13 +1076,22 @@ __device__ inline float score_block_any(const Params& p, const float* q_s, int b
   for (int d0 = 0; d0 < hd; d0 += kBatch) {
     float rv[kBatch];
 #pragma unroll
-    for (int k = 0; k < kBatch; ++k)
-      rv[k] = d0 + k < hd ? load_stream_f32(r + static_cast<int64_t>(d0 + k) * stride) : 0.0f;
+    for (int c = 0; c < kBatch; c += kStep) {
+      if (d0 + c < hd) {
 #pragma unroll
-    for (int k = 0; k < kBatch; ++k) {
-      if (d0 + k >= hd) break;
+        for (int k = 0; k < kStep; ++k) rv[c + k] = load_stream_f32(r + static_cast<int64_t>(d0 + c + k) * stride);
+      }
+    }
 #pragma unroll
-      for (int j = 0; j < G; ++j) dot[j] = dot[j] + q_s[j * hd + d0 + k] * rv[k];
+    for (int c = 0; c < kBatch; c += kStep) {
+      if (d0 + c < hd) {
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int k = 0; k < kStep; ++k) {
+#pragma unroll
+          for (int j = 0; j < G; ++j) dot[j] = dot[j] + q_s[j * hd + d0 + c + k] * rv[c + k];
+        }
+      }
     }
   }
   const float heads_f = static_cast<float>(G);
@@ -1001,7 +1102,7 @@ __device__ inline float score_block_any(const Params& p, const float* q_s, int b
 }
 
 template <int G, int LPR, bool F16, bool SPLIT>
-__global__ __launch_bounds__(kThreads) void decode_kernel_rows(const Params p, int hd) {
+__global__ __launch_bounds__(kThreads, G == 4 && LPR > 8 ? 2 : 4) void decode_kernel_rows(const Params p, int hd) {
   static_assert(G <= kRowsMaxG, "1, 2 or 4 query heads per KV head");
   using State = rows::RowsState<G, LPR>;
   const int g = blockIdx.x;
@@ -1220,7 +1321,13 @@ __global__ __launch_bounds__(kThreads) void decode_kernel_staged(const Params p)
 #pragma unroll
     for (int i = 0; i < kQLoads; ++i) q_t[(tid % D) * G + tid / D + i * (kThreads / D)] = q_entry[i];
     __syncthreads();
-    sel::score_blocks_vec<GR, 2, kThreads>(a, q_t, n, keys, nullptr, tid);
+    // one block per lane up to 512 blocks (two per lane would leave waves
+    // without blocks), else two
+    if (n <= kThreads) {
+      sel::score_blocks_t<GR, kThreads>(a, q_t, n, keys, nullptr);
+    } else {
+      sel::score_blocks_vec<GR, 2, kThreads>(a, q_t, n, keys, nullptr, tid);
+    }
   }
   if (ONLINE && deferred && tail_page >= 0) {
     // the group's query rows of this step to the ring (read by later seals)

@@ -58,12 +58,12 @@ __device__ inline void load_query(const ScoreArgs& a, float* q_s) {
 
 constexpr int kScoreBatch = 64;
 
-// Issue the first batch of representative loads of block `blk` (d 0..63 of
+// Issue a batch of representative loads of block `blk` (d0 .. d0 + 63 of
 // the group's first representative row) before the query is in LDS, so the
 // representative stream starts while the caller does other work.
-__device__ inline void score_prefetch(const ScoreArgs& a, int blk, float (&rv)[kScoreBatch]) {
+__device__ inline void score_prefetch(const ScoreArgs& a, int blk, float (&rv)[kScoreBatch], int d0 = 0) {
   const int rh = a.rep_heads == a.query_heads ? a.h_first : a.h_first / a.group;
-  const float* r = a.reps + (static_cast<int64_t>(a.b) * a.rep_heads + rh) * D * a.rep_stride + blk;
+  const float* r = a.reps + ((static_cast<int64_t>(a.b) * a.rep_heads + rh) * D + d0) * a.rep_stride + blk;
 #pragma unroll
   for (int k = 0; k < kScoreBatch; ++k) rv[k] = load_stream_f32(r + static_cast<int64_t>(k) * a.rep_stride);
 }
@@ -364,6 +364,35 @@ __device__ inline void row_dots(const ScoreArgs& a, const float* q_t, int blk0, 
     dot_vecs<GR, NB, KB>(q_t, qoff, hps, h0, d0, ra, dot);
     if (d0 + 2 * KB < D) load_vecs<NB, KB>(r, stride, d0 + 2 * KB, ra);
     dot_vecs<GR, NB, KB>(q_t, qoff, hps, h0, d0 + KB, rb, dot);
+  }
+}
+
+// row_dots() of one block with the whole representative row loaded at once:
+// one round trip to memory where few workgroups run and nothing else hides
+// it (in two batches of 32 twice over, 64 blocks took 10.5 us).  The products
+// go in steps of 16 rows, whose query reads stay behind the step before
+// (all 128 read ahead would not fit the registers).
+template <int GR>
+__device__ inline void row_dots_at_once(const ScoreArgs& a, const float* q_t, int blk, int h0, float (&dot)[GR][1]) {
+  constexpr int kStep = 16;
+  const int h = a.h_first + h0;
+  const int rh = a.rep_heads == a.query_heads ? h : h / a.group;
+  const float* r = a.reps + (static_cast<int64_t>(a.b) * a.rep_heads + rh) * D * a.rep_stride + blk;
+  float rv[D];
+#pragma unroll
+  for (int d = 0; d < D; ++d) rv[d] = load_stream_f32(r + static_cast<int64_t>(d) * a.rep_stride);
+#pragma unroll
+  for (int j = 0; j < GR; ++j) dot[j][0] = 0.0f;
+#pragma unroll
+  for (int d0 = 0; d0 < D; d0 += kStep) {
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int k = 0; k < kStep; ++k) {
+      float qv[GR];
+      read_q_t<GR>(q_t + (d0 + k) * a.heads_per_sel + h0, qv);
+#pragma unroll
+      for (int j = 0; j < GR; ++j) dot[j][0] = dot[j][0] + qv[j] * rv[d0 + k];
+    }
   }
 }
 
@@ -671,7 +700,8 @@ __device__ inline int compact_ids_wave(const uint32_t* keys, int n, const Budget
 // T takes bit b when at least k candidates have keys >= T | 2^b, counted with
 // one wave ballot per register and scalar popcounts.  Every test value is
 // >= 1, so the masked zeros are never counted and a candidate whose key is 0
-// is ranked correctly.  The take and the ascending compaction are those of
+// is ranked correctly.  The bits end once exactly k candidates remain (after
+// about 20 of 32 on real scores).  The take and the ascending compaction are those of
 // compact_ids_wave.
 //
 // The compares of eight (or four) registers are issued back to back (one asm
@@ -736,12 +766,19 @@ __device__ inline int select_ids_wave_regs(const uint32_t* keys, int n, const Bu
   int equal_take = 0;
   if (dynamic) {
     uint32_t t = 0;
-    for (int bit = 31; bit >= 0; --bit) {
+    bool exact = false;  // exactly k candidates at or above t: the lower bits cannot change the set
+    for (int bit = 31; bit >= 0 && !exact; --bit) {
       const uint32_t c = t | (1u << bit);
-      if (count_at_least<NC>(kr, c) >= bs.k) t = c;
+      const int at_least = count_at_least<NC>(kr, c);
+      if (at_least >= bs.k) t = c;
+      exact = at_least == bs.k;
     }
-    threshold = t;
-    equal_take = bs.k - (t == 0xffffffffu ? 0 : count_at_least<NC>(kr, t + 1u));
+    if (exact) {
+      threshold = t - 1u;  // all above it, none of those equal to it
+    } else {
+      threshold = t;
+      equal_take = bs.k - (t == 0xffffffffu ? 0 : count_at_least<NC>(kr, t + 1u));
+    }
   }
   const uint64_t below = (1ull << lane) - 1ull;
   int taken_eq = 0, written = 0;
