@@ -650,7 +650,9 @@ static size_t step_min_bytes(const sa_paged_kv* kv, int32_t splits) {
 }
 
 static size_t split_step_bytes(const sa_paged_kv* kv, int32_t splits) {
-  return static_cast<size_t>(kv->batch) * kv->query_heads * splits * sa::part_stride(kv->head_dim) * sizeof(float);
+  const size_t records =
+      static_cast<size_t>(kv->batch) * kv->query_heads * splits * sa::part_stride(kv->head_dim) * sizeof(float);
+  return (records + 255) / 256 * 256;
 }
 
 size_t sa_hip_decode_step_workspace_bytes(const sa_paged_kv* kv, int32_t splits) {
@@ -658,7 +660,30 @@ size_t sa_hip_decode_step_workspace_bytes(const sa_paged_kv* kv, int32_t splits)
   const size_t need = step_min_bytes(kv, splits);
   if (kv->kv_heads <= 0 || kv->query_heads <= 0 || kv->head_dim <= 0) return need;
   const int32_t cap = sa::split_step_cap(kv->batch, kv->query_heads, kv->kv_heads, kv->head_dim);
-  return std::max(need, arrive_bytes(kv->batch) + split_step_bytes(kv, cap));
+  return std::max(need,
+                  arrive_bytes(kv->batch) + split_step_bytes(kv, cap) + split_scores_bytes(kv, kv->query_heads));
+}
+
+// Whether the step after append + seal runs as a scoring launch and a launch of
+// several workgroups per list that select from the scores, attend and merge
+// (f.scores and *splits set): fewer lists than compute units, as for
+// sa_hip_score_select_split_preferred() (with a list per compute unit its
+// scoring launch is no faster), or a head_dim other than 128 (whose scoring is
+// always a launch of its own); the records, then the scores in the workspace.
+static bool scored_split_step(const sa_paged_kv* kv, sa::SelectAttendLaunch* f, void* records, size_t records_bytes,
+                              int32_t* splits) {
+  if (static_cast<int64_t>(kv->batch) * f->select_groups >= sa::compute_units() &&
+      !sa::general_head_dim(kv->head_dim))
+    return false;
+  const size_t sb = split_scores_bytes(kv, f->select_groups);
+  f->append = 0;
+  f->scores = static_cast<const float*>(records);  // (set: asks for the form with scores)
+  int32_t s = sa::split_step_splits(*f);
+  while (s > 0 && split_step_bytes(kv, s) + sb > records_bytes) --s;
+  f->scores = s < 1 ? nullptr
+                    : reinterpret_cast<const float*>(static_cast<uint8_t*>(records) + split_step_bytes(kv, s));
+  *splits = s;
+  return s >= 1;
 }
 
 // The step with several workgroups per list, where it applies and the records
@@ -731,6 +756,14 @@ static int decode_step_run(const sa_paged_kv* kv, const float* k, const float* v
       return fail(SA_HIP_EINVAL, "%s: workspace too small for the records and scores", op);
     l.scores = reinterpret_cast<float*>(static_cast<uint8_t*>(records) + rb);
     if (int e = lifecycle_common(kv, k, v, k16, v16, local_tokens, 1, status, stream, op, query, nullptr)) return e;
+    sa::SelectAttendLaunch f = step_launch();
+    int32_t s = 0;
+    if (!clear_arrive && scored_split_step(kv, &f, records, records_bytes, &s)) {
+      l.scores = const_cast<float*>(f.scores);
+      if (int e = check_hip(sa::launch_scores(l, as_stream(stream)), "decode_step: scoring launch")) return e;
+      return check_hip(sa::launch_split_step(f, static_cast<float*>(records), s, as_stream(stream)),
+                       "decode_step launch");
+    }
     if (int e = check_hip(sa::launch_score_select_split(l, as_stream(stream)), "decode_step: score_select launch"))
       return e;
     return attention_common(kv, query, selected, counts, params->select_groups, params->sel_stride, scale, out,
@@ -755,6 +788,13 @@ static int decode_step_run(const sa_paged_kv* kv, const float* k, const float* v
       f.append = 0;
       const int e = try_split_step(kv, f, records, records_bytes, stream, &done);
       if (e || done) return e;
+    }
+    int32_t s = 0;
+    if (!clear_arrive && scored_split_step(kv, &f, records, records_bytes, &s)) {
+      l.scores = const_cast<float*>(f.scores);
+      if (int e = check_hip(sa::launch_scores(l, as_stream(stream)), "decode_step: scoring launch")) return e;
+      return check_hip(sa::launch_split_step(f, static_cast<float*>(records), s, as_stream(stream)),
+                       "decode_step launch");
     }
     // few lists: the split selection (scoring spread over the device, the
     // scores after the records) where the scratch holds the scores; the same

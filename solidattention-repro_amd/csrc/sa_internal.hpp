@@ -87,6 +87,8 @@ struct SelectLaunch {
 hipError_t launch_score_select(const SelectLaunch& s, hipStream_t stream);
 // scoring over chunks of 256 blocks into s.scores, then selection from them
 hipError_t launch_score_select_split(const SelectLaunch& s, hipStream_t stream);
+// Its scoring launch alone.
+hipError_t launch_scores(const SelectLaunch& s, hipStream_t stream);
 // lists split into chunks of 512 blocks, one launch: workspace of
 // score_select_chunked_workspace_bytes(), its arrival counters zeroed once
 // (each launch leaves them at zero); needs 16-byte representative loads
@@ -189,6 +191,9 @@ struct SelectAttendLaunch {
   int32_t window;
   int32_t topk;
   float seal_scale;
+  // launch_split_step, append 0: the lists' scores ([batch][select_groups]
+  // [rep_stride]) from launch_scores()
+  const float* scores;
 };
 
 // The fused kernels: 1-2 query heads per KV head (registers), or 4 (LDS-staged

@@ -636,7 +636,7 @@ void launch_rows(const Params& p, int batch, hipStream_t stream) {
   }
 }
 
-hipError_t launch_score_select_split(const SelectLaunch& s, hipStream_t stream) {
+hipError_t launch_scores(const SelectLaunch& s, hipStream_t stream) {
   const Params p = make_params(s);
   const int chunks = (s.rep_stride + kChunkBlocks - 1) / kChunkBlocks;
   const dim3 grid(s.select_groups, s.batch, chunks);
@@ -668,8 +668,13 @@ hipError_t launch_score_select_split(const SelectLaunch& s, hipStream_t stream) 
       default: return hipErrorInvalidValue;
     }
   }
-  const hipError_t e0 = hipGetLastError();
+  return hipGetLastError();
+}
+
+hipError_t launch_score_select_split(const SelectLaunch& s, hipStream_t stream) {
+  const hipError_t e0 = launch_scores(s, stream);
   if (e0 != hipSuccess) return e0;
+  const Params p = make_params(s);
   // enough whole waves for every block of the row at kRegsKeys per thread,
   // at most 16 (the kernel takes twice as many per thread beyond 4096 blocks
   // and refuses the blocks past 8192)

@@ -76,6 +76,10 @@ struct Params {
   float* part;
   int32_t splits;
   int32_t field_bits;
+  // split launches: the lists' scores from an earlier launch ([list][rep_stride];
+  // null: scored here), and KV heads per list (1 where scored here)
+  const float* scores;
+  int32_t kv_per_sel;
 };
 
 __device__ inline int64_t table_page(const attn::PoolView& v, int b, int64_t logical) {
@@ -303,6 +307,40 @@ __device__ inline void finish_split(const Params& p, int b, int g, int hd, int64
     }
     p.arrive[b] = 0;
   }
+}
+
+// A list's scores as block keys in LDS.
+__device__ inline void keys_from_scores(const Params& p, int64_t list, int n, uint32_t* keys) {
+  const float* row = p.scores + list * p.rep_stride;
+#pragma unroll 8
+  for (int i = threadIdx.x; i < n; i += kThreads) keys[i] = sel::order_key(row[i]);
+}
+
+// The selection of a long list by the whole workgroup: wave 0 alone holds up
+// to 1024 keys in registers and takes the LDS histograms beyond, about 3 us a
+// thousand keys.  ids (may be the keys' own array) and, for the workgroup that
+// writes them, out_ids get the ascending block ids; returns the count.  Every
+// thread calls it, keys complete; the ids are visible on return.
+constexpr int kWideKeys = 8;
+typedef sel::RegsSelectSmem<kThreads, 4> WideSmem;
+
+__device__ inline bool selects_wide(int n, const sel::Budget& bs) {
+  return !bs.bad && !bs.take_all && n > 16 * kWave && n <= kWideKeys * kThreads;
+}
+
+__device__ inline int select_wide(const uint32_t* keys, int n, const sel::Budget& bs, int32_t* ids, int32_t* out_ids,
+                                  int sel_stride, WideSmem& sm) {
+  sel::clear_regs_select(sm);
+  __syncthreads();
+  const int count = n <= 4 * kThreads
+                        ? sel::select_from_keys_regs<kThreads, 4, 4>(keys, n, bs, ids, sel_stride, sm)
+                        : sel::select_from_keys_regs<kThreads, kWideKeys, 4>(keys, n, bs, ids, sel_stride, sm);
+  __syncthreads();
+  if (out_ids) {
+    for (int i = threadIdx.x; i < count; i += kThreads) out_ids[i] = ids[i];
+    __syncthreads();  // before the ids are replaced by their pages
+  }
+  return count;
 }
 
 // ---- the planned page walk (both fused kernels) ------------------------------
@@ -643,7 +681,9 @@ __device__ inline void decode_body(const Params& p, const Prod& qp) {
   __shared__ ClaimSmem cl;
   __shared__ uint32_t s_old;  // (SPLIT)
 
-  const int64_t out_row = static_cast<int64_t>(b) * p.v.kv_heads + g;
+  const int64_t out_row = SPLIT ? static_cast<int64_t>(b) * (p.v.kv_heads / p.kv_per_sel) + g / p.kv_per_sel
+                                : static_cast<int64_t>(b) * p.v.kv_heads + g;
+  const bool writes_ids = !SPLIT || (z == 0 && g % p.kv_per_sel == 0);
   // the group's query rows, loaded at entry (their latency overlaps the append)
   const float* q_group = p.query + (static_cast<int64_t>(b) * p.query_heads + g * G) * D;
   float q_entry = 0.0f;
@@ -689,8 +729,8 @@ __device__ inline void decode_body(const Params& p, const Prod& qp) {
   // SPLIT: lanes tid and tid + 256 share a block (see score_halves()) and each
   // prefetches its half
   constexpr int kHalf = kThreads / 2;
-  const bool have_pre = kPrefetch && n >= 0 && n <= p.rep_stride &&
-                        n <= kMaxSelectBlocks && (SPLIT ? tid % kHalf : tid) < n;
+  const bool have_pre = kPrefetch && n >= 0 && n <= p.rep_stride && n <= kMaxSelectBlocks &&
+                        (SPLIT ? tid % kHalf : tid) < n && !(SPLIT && p.scores);
   float pre[sel::kScoreBatch];
   if (have_pre) sel::score_prefetch(a, SPLIT ? tid % kHalf : tid, pre, SPLIT ? tid / kHalf * sel::kScoreBatch : 0);
 
@@ -716,7 +756,9 @@ __device__ inline void decode_body(const Params& p, const Prod& qp) {
            : sel::Budget{0, 0, 0, false, true};
   const Forced fb = forced_blocks(bs, n);
   const int32_t early = wave == kWaves - 1 ? early_page(p, b, n, fb, lane) : -1;
-  if (n_ok && !bs.take_all) {  // (a budget that takes every block needs no scores)
+  if (SPLIT && p.scores) {
+    if (n_ok && !bs.take_all) keys_from_scores(p, out_row, n, keys);
+  } else if (n_ok && !bs.take_all) {  // (a budget that takes every block needs no scores)
     if (!kProd && tid < G * D) q_s[tid] = q_entry;
     __syncthreads();
     if constexpr (SPLIT) {
@@ -746,17 +788,26 @@ __device__ inline void decode_body(const Params& p, const Prod& qp) {
 
   // ---- 3. select (wave 0) and walk (every wave, planned positions) -------------
   int32_t* late = reinterpret_cast<int32_t*>(keys);  // the selected ids, then the late pages
+  int wide_count = -1;
+  if constexpr (SPLIT) {
+    __shared__ __align__(16) WideSmem wide;
+    if (p.scores && n_ok && selects_wide(n, bs))
+      wide_count = select_wide(keys, n, bs, late, writes_ids ? p.selected + out_row * p.sel_stride : nullptr,
+                               p.sel_stride, wide);
+  }
   if (wave == 0) {
     int count = 0;
     if (!n_ok || bs.bad) {
       if (lane == 0) {
         flag_status(p.v.status, n_ok ? kStatusBadBudget : kStatusCapacity);
-        if (z == 0) p.counts[out_row] = 0;
+        if (writes_ids) p.counts[out_row] = 0;
       }
     } else {
-      count = sel::select_ids_wave(keys, n, bs, hist, z == 0 ? p.selected + out_row * p.sel_stride : nullptr,
-                                   p.sel_stride, late);
-      if (lane == 0 && z == 0) p.counts[out_row] = count;
+      count = wide_count >= 0 ? wide_count
+                              : sel::select_ids_wave(keys, n, bs, hist,
+                                                     writes_ids ? p.selected + out_row * p.sel_stride : nullptr,
+                                                     p.sel_stride, late);
+      if (lane == 0 && writes_ids) p.counts[out_row] = count;
     }
     list_late(p, b, cl, late, kMaxSelectBlocks, count, fb, wn, tail_pages, lane);
   }
@@ -1068,7 +1119,8 @@ template <int G>
 __device__ inline float score_block_any(const Params& p, const float* q_s, int b, int g, int hd, int blk) {
   constexpr int kBatch = 64;  // (a whole row at head_dim 64: one round trip to memory)
   constexpr int kStep = 8;    // head_dim is a multiple of 8
-  const int64_t stride = p.rep_stride;
+  int64_t stride = p.rep_stride;
+  asm volatile("" : "+s"(stride));  // (or 64 row offsets are kept across the lane's blocks, and spill)
   const float* r = p.reps + (static_cast<int64_t>(b) * p.rep_heads + g) * hd * stride + blk;
   float dot[G];
 #pragma unroll
@@ -1101,7 +1153,7 @@ __device__ inline float score_block_any(const Params& p, const float* q_s, int b
   return score;
 }
 
-template <int G, int LPR, bool F16, bool SPLIT>
+template <int G, int LPR, bool APPEND, bool F16, bool SPLIT>
 __global__ __launch_bounds__(kThreads, G == 4 && LPR > 8 ? 2 : 4) void decode_kernel_rows(const Params p, int hd) {
   static_assert(G <= kRowsMaxG, "1, 2 or 4 query heads per KV head");
   using State = rows::RowsState<G, LPR>;
@@ -1120,15 +1172,19 @@ __global__ __launch_bounds__(kThreads, G == 4 && LPR > 8 ? 2 : 4) void decode_ke
   __shared__ float w_acc[kWaves][G][LPR * 8];
   __shared__ uint32_t s_old;  // (SPLIT)
 
-  const int64_t out_row = static_cast<int64_t>(b) * p.v.kv_heads + g;
+  const int64_t out_row = SPLIT ? static_cast<int64_t>(b) * (p.v.kv_heads / p.kv_per_sel) + g / p.kv_per_sel
+                                : static_cast<int64_t>(b) * p.v.kv_heads + g;
+  const bool writes_ids = !SPLIT || (z == 0 && g % p.kv_per_sel == 0);
   const float* q_group = p.query + (static_cast<int64_t>(b) * p.query_heads + g * G) * hd;
   for (int e = tid; e < G * hd; e += kThreads) q_s[e] = q_group[e];
   int64_t len = p.seq_len[b];
   int n = p.sealed[b];
 
   SeqCommit commit{};
-  commit.gen = p.generation ? p.generation[b] : 0;
-  commit.appended = append_seal_head_any<F16>(p, b, g, hd, len, n, commit.added);
+  if (APPEND) {
+    commit.gen = p.generation ? p.generation[b] : 0;
+    commit.appended = append_seal_head_any<F16>(p, b, g, hd, len, n, commit.added);
+  }
   if (!SPLIT && tid == 0) commit.arrived = atomicAdd(&p.arrive[b], 1);
 
   State st;
@@ -1142,7 +1198,9 @@ __global__ __launch_bounds__(kThreads, G == 4 && LPR > 8 ? 2 : 4) void decode_ke
   const Forced fb = forced_blocks(bs, n);
   const int32_t early = wave == kWaves - 1 ? early_page(p, b, n, fb, lane) : -1;
   __syncthreads();  // the query rows, and the representatives this workgroup sealed
-  if (n_ok && !bs.take_all) {  // (a budget that takes every block needs no scores)
+  if (SPLIT && p.scores) {
+    if (n_ok && !bs.take_all) keys_from_scores(p, out_row, n, keys);
+  } else if (n_ok && !bs.take_all) {  // (a budget that takes every block needs no scores)
     for (int blk = tid; blk < n; blk += kThreads) keys[blk] = sel::order_key(score_block_any<G>(p, q_s, b, g, hd, blk));
   }
   if (wave == kWaves - 1) cl.early[lane] = early;
@@ -1160,17 +1218,26 @@ __global__ __launch_bounds__(kThreads, G == 4 && LPR > 8 ? 2 : 4) void decode_ke
 
   // ---- select (wave 0) and walk (every wave, planned positions) -------------
   int32_t* late = reinterpret_cast<int32_t*>(keys);
+  int wide_count = -1;
+  if constexpr (SPLIT) {
+    __shared__ __align__(16) WideSmem wide;
+    if (p.scores && n_ok && selects_wide(n, bs))
+      wide_count = select_wide(keys, n, bs, late, writes_ids ? p.selected + out_row * p.sel_stride : nullptr,
+                               p.sel_stride, wide);
+  }
   if (wave == 0) {
     int count = 0;
     if (!n_ok || bs.bad) {
       if (lane == 0) {
         flag_status(p.v.status, n_ok ? kStatusBadBudget : kStatusCapacity);
-        if (z == 0) p.counts[out_row] = 0;
+        if (writes_ids) p.counts[out_row] = 0;
       }
     } else {
-      count = sel::select_ids_wave(keys, n, bs, hist, z == 0 ? p.selected + out_row * p.sel_stride : nullptr,
-                                   p.sel_stride, late);
-      if (lane == 0 && z == 0) p.counts[out_row] = count;
+      count = wide_count >= 0 ? wide_count
+                              : sel::select_ids_wave(keys, n, bs, hist,
+                                                     writes_ids ? p.selected + out_row * p.sel_stride : nullptr,
+                                                     p.sel_stride, late);
+      if (lane == 0 && writes_ids) p.counts[out_row] = count;
     }
     list_late(p, b, cl, late, kMaxSelectBlocks, count, fb, wn, tail_pages, lane);
   }
@@ -1214,7 +1281,7 @@ __global__ __launch_bounds__(kThreads, G == 4 && LPR > 8 ? 2 : 4) void decode_ke
     if constexpr (SPLIT) store_record(split_record(p, b, g, z, G, h, hd), d, mx, lw, aw);
     else p.out[(static_cast<int64_t>(b) * p.query_heads + g * G + h) * hd + d] = lw > 0.0f ? aw / lw : 0.0f;
   }
-  if constexpr (SPLIT) finish_split<G, true>(p, b, g, hd, len, n, commit, &s_old);
+  if constexpr (SPLIT) finish_split<G, APPEND>(p, b, g, hd, len, n, commit, &s_old);
   else if (tid == 0) commit_sequence(p, b, len, n, commit);
 }
 
@@ -1263,7 +1330,9 @@ __global__ __launch_bounds__(kThreads) void decode_kernel_staged(const Params p)
   float* pbuf = pbuf_s + wave * kPbufFloats;
   const float* q_group = p.query + (static_cast<int64_t>(b) * p.query_heads + g * G) * D;
 
-  const int64_t out_row = static_cast<int64_t>(b) * p.v.kv_heads + g;
+  const int64_t out_row = SPLIT ? static_cast<int64_t>(b) * (p.v.kv_heads / p.kv_per_sel) + g / p.kv_per_sel
+                                : static_cast<int64_t>(b) * p.v.kv_heads + g;
+  const bool writes_ids = !SPLIT || (z == 0 && g % p.kv_per_sel == 0);
   // the group's query rows, loaded at entry (their latency overlaps the append)
   constexpr int kQLoads = G * D / kThreads;
   float q_entry[kQLoads];
@@ -1306,7 +1375,9 @@ __global__ __launch_bounds__(kThreads) void decode_kernel_staged(const Params p)
            : sel::Budget{0, 0, 0, false, true};
   const Forced fb = forced_blocks(bs, n);
   const int32_t early = wave == kWaves - 1 ? early_page(p, b, n, fb, lane) : -1;
-  if (n_ok && !bs.take_all) {  // (a budget that takes every block needs no scores)
+  if (SPLIT && p.scores) {
+    if (n_ok && !bs.take_all) keys_from_scores(p, out_row, n, keys);
+  } else if (n_ok && !bs.take_all) {  // (a budget that takes every block needs no scores)
     sel::ScoreArgs a{};
     a.query = p.query;
     a.reps = p.reps;
@@ -1359,6 +1430,14 @@ __global__ __launch_bounds__(kThreads) void decode_kernel_staged(const Params p)
   __syncthreads();  // keys, the early pages and the flag visible
 
   // ---- 3. select (wave 0) and walk (every wave, planned positions) -------------
+  int wide_count = -1;
+  if constexpr (SPLIT) {
+    // (page slots 4 and 5: the keys reach into 0 and 1, no wave walks yet)
+    static_assert(sizeof(WideSmem) <= 2 * kSlotBytes, "the wide selection fits two page slots");
+    if (p.scores && n_ok && selects_wide(n, bs))
+      wide_count = select_wide(keys, n, bs, late_ids, writes_ids ? p.selected + out_row * p.sel_stride : nullptr,
+                               p.sel_stride, *reinterpret_cast<WideSmem*>(smem + 4 * kSlotBytes));
+  }
   if (wave == 0) {
     if (deferred) {
       if (tail_page >= 0) store_token_quad(p, tail_page, len - 1, g, lane, token);
@@ -1368,12 +1447,14 @@ __global__ __launch_bounds__(kThreads) void decode_kernel_staged(const Params p)
     if (!n_ok || bs.bad) {
       if (lane == 0) {
         flag_status(p.v.status, n_ok ? kStatusBadBudget : kStatusCapacity);
-        if (z == 0) p.counts[out_row] = 0;
+        if (writes_ids) p.counts[out_row] = 0;
       }
     } else {
-      count = sel::select_ids_wave(keys, n, bs, hist, z == 0 ? p.selected + out_row * p.sel_stride : nullptr,
-                                   p.sel_stride, late_ids);
-      if (lane == 0 && z == 0) p.counts[out_row] = count;
+      count = wide_count >= 0 ? wide_count
+                              : sel::select_ids_wave(keys, n, bs, hist,
+                                                     writes_ids ? p.selected + out_row * p.sel_stride : nullptr,
+                                                     p.sel_stride, late_ids);
+      if (lane == 0 && writes_ids) p.counts[out_row] = count;
     }
     list_late(p, b, cl, late_ids, kStagedIds + kTailPages, count, fb, wn, tail_pages, lane);
   }
@@ -1487,8 +1568,8 @@ hipError_t launch_shared(const Params& p, int batch, hipStream_t stream) {
 }
 
 // ---- the step with several workgroups per list ----------------------------------
-// Every workgroup of a list scores all of it, so long lists are left to the
-// launches that share the scores.
+// Every workgroup of a list scores all of it; longer lists, and groups of
+// several KV heads, take their scores from a scoring launch (s.scores).
 constexpr int kMaxSplitStepBlocks = 1024;
 
 // Bits of a KV head's field in a sequence's 32-bit arrival counter.
@@ -1510,11 +1591,19 @@ int32_t split_step_cap(int32_t batch, int32_t query_heads, int32_t kv_heads, int
 }
 
 int32_t split_step_splits(const SelectAttendLaunch& s) {
-  if (s.ring || s.kv_heads <= 0 || s.rep_stride > kMaxSplitStepBlocks || split_field_bits(s.kv_heads) < 1) return 0;
+  if (s.ring || s.kv_heads <= 0 || split_field_bits(s.kv_heads) < 1) return 0;
   const int hd = s.head_dim > 0 ? s.head_dim : kHeadDim;
   const int group = s.query_heads / s.kv_heads;
   const bool shared = s.select_groups != s.kv_heads;
-  if (hd != kHeadDim) {
+  if (s.scores) {
+    if (s.append || s.select_groups <= 0 || s.kv_heads % s.select_groups != 0) return 0;
+    if (hd != kHeadDim ? hd > rows::kMaxHeadDim || hd % 8 != 0 || (group != 1 && group != 2 && group != 4)
+                       : group >= 4 && s.sel_stride > kStagedIds)
+      return 0;
+    if (group != 1 && group != 2 && group != 4 && group != 8) return 0;
+  } else if (s.rep_stride > kMaxSplitStepBlocks) {
+    return 0;
+  } else if (hd != kHeadDim) {
     if (!s.append || !select_attend_rows_supported(s.query_heads, s.kv_heads, s.rep_heads, s.select_groups, hd))
       return 0;
   } else if (shared) {
@@ -1566,23 +1655,23 @@ bool select_attend_rows_supported(int32_t query_heads, int32_t kv_heads, int32_t
          head_dim <= rows::kMaxHeadDim && head_dim != kHeadDim;
 }
 
-template <int LPR, bool F16, bool SPLIT>
+template <int LPR, bool F16, bool SPLIT, bool APPEND>
 hipError_t launch_rows_step(const Params& p, int batch, int hd, hipStream_t stream) {
   const dim3 grid(p.v.kv_heads, batch, SPLIT ? p.splits : 1), block(kThreads);
   switch (p.query_heads / p.v.kv_heads) {
-    case 1: hipLaunchKernelGGL((decode_kernel_rows<1, LPR, F16, SPLIT>), grid, block, 0, stream, p, hd); break;
-    case 2: hipLaunchKernelGGL((decode_kernel_rows<2, LPR, F16, SPLIT>), grid, block, 0, stream, p, hd); break;
-    default: hipLaunchKernelGGL((decode_kernel_rows<4, LPR, F16, SPLIT>), grid, block, 0, stream, p, hd); break;
+    case 1: hipLaunchKernelGGL((decode_kernel_rows<1, LPR, APPEND, F16, SPLIT>), grid, block, 0, stream, p, hd); break;
+    case 2: hipLaunchKernelGGL((decode_kernel_rows<2, LPR, APPEND, F16, SPLIT>), grid, block, 0, stream, p, hd); break;
+    default: hipLaunchKernelGGL((decode_kernel_rows<4, LPR, APPEND, F16, SPLIT>), grid, block, 0, stream, p, hd); break;
   }
   return hipGetLastError();
 }
 
-template <bool F16, bool SPLIT = false>
+template <bool F16, bool SPLIT = false, bool APPEND = true>
 hipError_t launch_rows_lpr(const Params& p, int batch, int hd, hipStream_t stream) {
   switch (rows::lanes_per_row(hd)) {
-    case 8: return launch_rows_step<8, F16, SPLIT>(p, batch, hd, stream);
-    case 16: return launch_rows_step<16, F16, SPLIT>(p, batch, hd, stream);
-    default: return launch_rows_step<32, F16, SPLIT>(p, batch, hd, stream);
+    case 8: return launch_rows_step<8, F16, SPLIT, APPEND>(p, batch, hd, stream);
+    case 16: return launch_rows_step<16, F16, SPLIT, APPEND>(p, batch, hd, stream);
+    default: return launch_rows_step<32, F16, SPLIT, APPEND>(p, batch, hd, stream);
   }
 }
 
@@ -1666,10 +1755,13 @@ hipError_t launch_split_step(const SelectAttendLaunch& s, float* records, int32_
   p.part = records;
   p.splits = splits;
   p.field_bits = split_field_bits(s.kv_heads);
+  p.scores = s.scores;
+  p.kv_per_sel = s.scores ? s.kv_heads / s.select_groups : 1;
+  if (hd != kHeadDim && !s.append) return launch_rows_lpr<false, true, false>(p, s.batch, hd, stream);
   if (hd != kHeadDim)
     return s.k16 ? launch_rows_lpr<true, true>(p, s.batch, hd, stream)
                  : launch_rows_lpr<false, true>(p, s.batch, hd, stream);
-  if (s.select_groups != s.kv_heads) {
+  if (s.select_groups != s.kv_heads && !s.scores) {
     if (!s.append) return launch_shared<false, false, true>(p, s.batch, stream);
     return s.k16 ? launch_shared<true, true, true>(p, s.batch, stream)
                  : launch_shared<true, false, true>(p, s.batch, stream);

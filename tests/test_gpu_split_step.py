@@ -17,7 +17,7 @@ from test_gpu_decode_sweep import SCALE, oracle_step
 
 pytestmark = pytest.mark.gpu
 
-# (query heads, KV heads, per-query-head reps, lengths, budget, init, local, local tokens)
+# (query heads, KV heads, per-query-head reps, lengths, budget, init, local, local tokens[, selection groups])
 CASES = [
     (1, 1, False, [32 * 40 + 31], 24, 1, 2, 0),
     (8, 8, False, [0, 31, 32 * 300 + 5], 64, 4, 8, 32),
@@ -28,13 +28,22 @@ CASES = [
     (8, 1, False, [32 * 70 + 31, 32 * 200, 17], 65, 4, 8, 0),
     (64, 8, False, [32 * 90 + 30, 32 * 6 + 31], 33, 4, 8, 0),
     (32, 4, True, [32 * 50 + 31], 300, 4, 8, 0),
+    # lists past 1024 blocks, and groups of several KV heads: scored by a launch of their own (the selection by one
+    # wave up to 1024 blocks, by the workgroup up to 4096, by one wave again beyond)
+    (4, 2, False, [32 * 1030 + 31, 32 * 1000 + 5, 77], 96, 4, 8, 0),
+    (8, 2, True, [32 * 1024 + 30, 32 * 1023 + 31], 40, 1, 2, 0),
+    (8, 1, False, [32 * 2100 + 31, 32 * 2048], 64, 4, 8, 32),
+    (1, 1, False, [32 * 4110, 32 * 4095 + 31], 33, 0, 1, 0),
+    (16, 4, False, [32 * 150 + 31, 0], 24, 1, 2, 0, 1),
+    (16, 8, False, [32 * 140 + 30], 16, 1, 2, 0, 2),
 ]
 
 
 @pytest.mark.parametrize("case_id", range(len(CASES)))
 @pytest.mark.parametrize("splits", [1, 2])
 def test_split_step(hip, case_id, splits):
-    hq, hkv, per_query, lengths, budget, init, local, local_tokens = CASES[case_id]
+    hq, hkv, per_query, lengths, budget, init, local, local_tokens = CASES[case_id][:8]
+    groups = CASES[case_id][8] if len(CASES[case_id]) > 8 else hkv
     print(f"case: {CASES[case_id]} splits={splits}", flush=True)
     batch = len(lengths)
     case = make_case(300 + case_id, batch, hq, hkv, lengths, rep_heads=hq if per_query else None,
@@ -51,15 +60,15 @@ def test_split_step(hip, case_id, splits):
         kd, vd = to_dev(k), to_dev(v)
         if step == 3:  # raw FP16 tokens
             kd, vd = (x.to(torch.float16).view(torch.uint16) for x in (kd, vd))
-        sel, cnt, out = hip.decode_step(kv, kd, vd, local_tokens, to_dev(case.query), hkv, budget, init, local, SCALE,
-                                        ws, splits=splits, status=st)
-        esel, ecnt, expect = oracle_step(case, k, v, c)
+        sel, cnt, out = hip.decode_step(kv, kd, vd, local_tokens, to_dev(case.query), groups, budget, init, local,
+                                        SCALE, ws, splits=splits, status=st)
+        esel, ecnt, expect = oracle_step(case, k, v, c, groups)
         torch.cuda.synchronize()
         assert int(st.item()) == 0, step
         assert np.array_equal(cnt.cpu().numpy(), ecnt), step
         got = sel.cpu().numpy()
         for b in range(batch):
-            for g in range(hkv):
+            for g in range(groups):
                 n = int(ecnt[b, g])
                 assert got[b, g, :n].tolist() == esel[b, g, :n].tolist(), (step, b, g)
         assert_close_2e3(out.cpu().numpy(), expect)
