@@ -1131,7 +1131,8 @@ __device__ inline float score_block_any(const Params& p, const float* q_s, int b
     for (int c = 0; c < kBatch; c += kStep) {
       if (d0 + c < hd) {
 #pragma unroll
-        for (int k = 0; k < kStep; ++k) rv[c + k] = load_stream_f32(r + static_cast<int64_t>(d0 + c + k) * stride);
+        for (int k = 0; k < kStep; ++k) rv[c + k] = load_stream_f32(r + k * stride);
+        r += kStep * stride;
       }
     }
 #pragma unroll
