@@ -741,7 +741,7 @@ def attention_contiguous(kv16, query, tokens, query_heads, kv_heads, scale, out=
     if out is None:
         out = torch.empty((query_heads, head_dim), dtype=torch.float32, device=query.device)
     nbytes = lib().sa_hip_contiguous_workspace_bytes(tokens, query_heads, kv_heads, head_dim)
-    ws = torch.zeros(max(nbytes // 4, 1), dtype=torch.float32, device=query.device)
+    ws = torch.empty(max(nbytes // 4, 1), dtype=torch.float32, device=query.device)  # written before it is read
     check(lib().sa_hip_attention_contiguous(_ptr(kv16), _ptr(query), tokens, query_heads, kv_heads, head_dim,
                                             C.c_float(scale), _ptr(out), _ptr(ws), nbytes, _stream(stream)),
           "attention_contiguous")
