@@ -696,14 +696,20 @@ static bool scored_split_step(const sa_paged_kv* kv, sa::SelectAttendLaunch* f, 
   return s >= 1;
 }
 
-// The step with several workgroups per list, where it applies and the records
-// fit (*done): one launch, or, with the online seal (f.append 0 by then), the
-// launch behind append + seal.
+// The splits of the step with several workgroups per list whose records fit
+// (0: it does not apply).
+static int32_t split_step_fit(const sa_paged_kv* kv, const sa::SelectAttendLaunch& f, size_t records_bytes) {
+  int32_t s = sa::split_step_splits(f);
+  while (s > 0 && split_step_bytes(kv, s) > records_bytes) --s;
+  return s;
+}
+
+// That step where it applies (*done): one launch, or, with the online seal
+// (f.append 0 by then), the launch behind append + seal.
 static int try_split_step(const sa_paged_kv* kv, const sa::SelectAttendLaunch& f, void* records,
                           size_t records_bytes, void* stream, bool* done) {
   *done = false;
-  int32_t s = sa::split_step_splits(f);
-  while (s > 0 && split_step_bytes(kv, s) > records_bytes) --s;
+  const int32_t s = split_step_fit(kv, f, records_bytes);
   if (s < 1) return SA_HIP_OK;
   *done = true;
   return check_hip(sa::launch_split_step(f, static_cast<float*>(records), s, as_stream(stream)),
@@ -782,6 +788,21 @@ static int decode_step_run(const sa_paged_kv* kv, const float* k, const float* v
   // (the online seal's one launch selects per KV group)
   const bool fused =
       sa_hip_select_attend_fused(kv, params, splits) && !(seal && params->select_groups != kv->kv_heads);
+  if (producer && !fused && !clear_arrive &&
+      sa::decode_step_qkv_supported(kv->query_heads, kv->kv_heads, params->select_groups, kv->head_dim)) {
+    // the producer's partial launch, then several workgroups per list that run
+    // its epilogue
+    const sa::SelectAttendLaunch f = step_launch();
+    const int32_t s = split_step_fit(kv, f, records_bytes);
+    if (s >= 1) {
+      sa::qkv::ReduceParams r;
+      if (int e = check_hip(sa::launch_qkv_partials(*producer, &r, as_stream(stream)),
+                            "decode_step: q/k/v partials launch"))
+        return e;
+      return check_hip(sa::launch_decode_step_qkv(f, r, as_stream(stream), static_cast<float*>(records), s),
+                       "decode_step launch");
+    }
+  }
   if (producer && !(fused && sa::decode_step_qkv_supported(kv->query_heads, kv->kv_heads, params->select_groups,
                                                            kv->head_dim)))
     if (int e = check_hip(sa::launch_qkv_project(*producer, as_stream(stream)), "decode_step: q/k/v producer launch"))

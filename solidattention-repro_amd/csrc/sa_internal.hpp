@@ -230,7 +230,9 @@ hipError_t launch_select_attend(const SelectAttendLaunch& s, hipStream_t stream)
 // per KV head, fp32 token, no online seal; r from launch_qkv_partials() with
 // rows == batch and r.q == s.query.
 bool decode_step_qkv_supported(int32_t query_heads, int32_t kv_heads, int32_t select_groups, int32_t head_dim);
-hipError_t launch_decode_step_qkv(const SelectAttendLaunch& s, const qkv::ReduceParams& r, hipStream_t stream);
+// records, splits: the form with several workgroups per list (launch_split_step).
+hipError_t launch_decode_step_qkv(const SelectAttendLaunch& s, const qkv::ReduceParams& r, hipStream_t stream,
+                                  float* records = nullptr, int32_t splits = 1);
 
 // InfLLM local-causal block representatives of a prefill (contiguous KV).
 struct RepresentativeLaunch {
