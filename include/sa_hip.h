@@ -318,9 +318,7 @@ int sa_hip_select_attend(const sa_paged_kv* kv, const float* query,
  * floats; used when the step runs as separate launches with few lists, and
  * at every head_dim other than 128), and at least as large as the counters
  * and the partial records of a one-launch step that spreads each list over
- * several workgroups.  A smaller workspace that holds the counters, the
- * split records and the scores is accepted (with fewer workgroups per list,
- * or separate launches).  The caller
+ * several workgroups.  The caller
  * zeroes it ONCE before the first call; every call leaves the counters at
  * zero again.  Calls sharing a workspace must not run concurrently. */
 size_t sa_hip_decode_step_workspace_bytes(const sa_paged_kv* kv,

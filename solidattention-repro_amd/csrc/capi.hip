@@ -652,12 +652,7 @@ static size_t split_scores_bytes(const sa_paged_kv* kv, int32_t select_groups) {
   return static_cast<size_t>(kv->batch) * select_groups * (kv->rep_stride > 0 ? kv->rep_stride : 0) * sizeof(float);
 }
 
-// What every step accepts (counters, the caller's split records, scores); the
-// workspace is sized for the records of the split step as well, which uses as
-// many splits as the workspace holds records for.
-static size_t step_min_bytes(const sa_paged_kv* kv, int32_t splits) {
-  return arrive_bytes(kv->batch) + split_records_bytes(kv, splits) + split_scores_bytes(kv, kv->query_heads);
-}
+// Records of the step with several workgroups per list.
 
 static size_t split_step_bytes(const sa_paged_kv* kv, int32_t splits) {
   const size_t records =
@@ -667,7 +662,8 @@ static size_t split_step_bytes(const sa_paged_kv* kv, int32_t splits) {
 
 size_t sa_hip_decode_step_workspace_bytes(const sa_paged_kv* kv, int32_t splits) {
   if (!kv || kv->batch <= 0) return 0;
-  const size_t need = step_min_bytes(kv, splits);
+  const size_t need =
+      arrive_bytes(kv->batch) + split_records_bytes(kv, splits) + split_scores_bytes(kv, kv->query_heads);
   if (kv->kv_heads <= 0 || kv->query_heads <= 0 || kv->head_dim <= 0) return need;
   const int32_t cap = sa::split_step_cap(kv->batch, kv->query_heads, kv->kv_heads, kv->head_dim);
   return std::max(need,
@@ -679,37 +675,27 @@ size_t sa_hip_decode_step_workspace_bytes(const sa_paged_kv* kv, int32_t splits)
 // (f.scores and *splits set): fewer lists than compute units, as for
 // sa_hip_score_select_split_preferred() (with a list per compute unit its
 // scoring launch is no faster), or a head_dim other than 128 (whose scoring is
-// always a launch of its own); the records, then the scores in the workspace.
-static bool scored_split_step(const sa_paged_kv* kv, sa::SelectAttendLaunch* f, void* records, size_t records_bytes,
-                              int32_t* splits) {
+// always a launch of its own); the records, then the scores in the workspace,
+// which is sized for both.
+static bool scored_split_step(const sa_paged_kv* kv, sa::SelectAttendLaunch* f, void* records, int32_t* splits) {
   if (static_cast<int64_t>(kv->batch) * f->select_groups >= sa::compute_units() &&
       !sa::general_head_dim(kv->head_dim))
     return false;
-  const size_t sb = split_scores_bytes(kv, f->select_groups);
   f->append = 0;
   f->scores = static_cast<const float*>(records);  // (set: asks for the form with scores)
-  int32_t s = sa::split_step_splits(*f);
-  while (s > 0 && split_step_bytes(kv, s) + sb > records_bytes) --s;
+  const int32_t s = sa::split_step_splits(*f);
   f->scores = s < 1 ? nullptr
                     : reinterpret_cast<const float*>(static_cast<uint8_t*>(records) + split_step_bytes(kv, s));
   *splits = s;
   return s >= 1;
 }
 
-// The splits of the step with several workgroups per list whose records fit
-// (0: it does not apply).
-static int32_t split_step_fit(const sa_paged_kv* kv, const sa::SelectAttendLaunch& f, size_t records_bytes) {
-  int32_t s = sa::split_step_splits(f);
-  while (s > 0 && split_step_bytes(kv, s) > records_bytes) --s;
-  return s;
-}
-
-// That step where it applies (*done): one launch, or, with the online seal
-// (f.append 0 by then), the launch behind append + seal.
-static int try_split_step(const sa_paged_kv* kv, const sa::SelectAttendLaunch& f, void* records,
-                          size_t records_bytes, void* stream, bool* done) {
+// The step with several workgroups per list where it applies (*done): one
+// launch, or, with the online seal (f.append 0 by then), the launch behind
+// append + seal.  The workspace is sized for the records.
+static int try_split_step(const sa::SelectAttendLaunch& f, void* records, void* stream, bool* done) {
   *done = false;
-  const int32_t s = split_step_fit(kv, f, records_bytes);
+  const int32_t s = sa::split_step_splits(f);
   if (s < 1) return SA_HIP_OK;
   *done = true;
   return check_hip(sa::launch_split_step(f, static_cast<float*>(records), s, as_stream(stream)),
@@ -763,7 +749,7 @@ static int decode_step_run(const sa_paged_kv* kv, const float* k, const float* v
     if (seal) return fail(SA_HIP_EINVAL, "%s: the online seal is built for head_dim %d", op, sa::kHeadDim);
     if (!clear_arrive) {
       bool done = false;
-      const int e = try_split_step(kv, step_launch(), records, records_bytes, stream, &done);
+      const int e = try_split_step(step_launch(), records, stream, &done);
       if (e || done) return e;
     }
     const size_t rb = split_records_bytes(kv, splits);
@@ -774,7 +760,7 @@ static int decode_step_run(const sa_paged_kv* kv, const float* k, const float* v
     if (int e = lifecycle_common(kv, k, v, k16, v16, local_tokens, 1, status, stream, op, query, nullptr)) return e;
     sa::SelectAttendLaunch f = step_launch();
     int32_t s = 0;
-    if (!clear_arrive && scored_split_step(kv, &f, records, records_bytes, &s)) {
+    if (!clear_arrive && scored_split_step(kv, &f, records, &s)) {
       l.scores = const_cast<float*>(f.scores);
       if (int e = check_hip(sa::launch_scores(l, as_stream(stream)), "decode_step: scoring launch")) return e;
       return check_hip(sa::launch_split_step(f, static_cast<float*>(records), s, as_stream(stream)),
@@ -793,7 +779,7 @@ static int decode_step_run(const sa_paged_kv* kv, const float* k, const float* v
     // the producer's partial launch, then several workgroups per list that run
     // its epilogue
     const sa::SelectAttendLaunch f = step_launch();
-    const int32_t s = split_step_fit(kv, f, records_bytes);
+    const int32_t s = sa::split_step_splits(f);
     if (s >= 1) {
       sa::qkv::ReduceParams r;
       if (int e = check_hip(sa::launch_qkv_partials(*producer, &r, as_stream(stream)),
@@ -811,17 +797,17 @@ static int decode_step_run(const sa_paged_kv* kv, const float* k, const float* v
     sa::SelectAttendLaunch f = step_launch();
     bool done = false;
     if (!seal && !clear_arrive) {
-      const int e = try_split_step(kv, f, records, records_bytes, stream, &done);
+      const int e = try_split_step(f, records, stream, &done);
       if (e || done) return e;
     }
     if (int e = lifecycle_common(kv, k, v, k16, v16, local_tokens, 1, status, stream, op, query, seal, arrive)) return e;
     if (seal && !clear_arrive) {
       f.append = 0;
-      const int e = try_split_step(kv, f, records, records_bytes, stream, &done);
+      const int e = try_split_step(f, records, stream, &done);
       if (e || done) return e;
     }
     int32_t s = 0;
-    if (!clear_arrive && scored_split_step(kv, &f, records, records_bytes, &s)) {
+    if (!clear_arrive && scored_split_step(kv, &f, records, &s)) {
       l.scores = const_cast<float*>(f.scores);
       if (int e = check_hip(sa::launch_scores(l, as_stream(stream)), "decode_step: scoring launch")) return e;
       return check_hip(sa::launch_split_step(f, static_cast<float*>(records), s, as_stream(stream)),
@@ -847,7 +833,7 @@ static int decode_step_run(const sa_paged_kv* kv, const float* k, const float* v
     // the shared selection's few workgroups, each list split over several
     bool done = false;
     if (sa::split_step_splits(f) > 1) {
-      const int e = try_split_step(kv, f, records, records_bytes, stream, &done);
+      const int e = try_split_step(f, records, stream, &done);
       if (e || done) return e;
     }
   }
@@ -881,7 +867,7 @@ static int decode_step_common(const sa_paged_kv* kv, const float* k, const float
                               float* out, void* workspace, size_t workspace_bytes, int32_t splits, int32_t* status,
                               void* stream, const char* op, const sa::QkvLaunch* producer = nullptr) {
   if (!kv || kv->batch <= 0) return fail(SA_HIP_EINVAL, "%s: null sa_paged_kv or empty batch", op);
-  const size_t need = step_min_bytes(kv, splits);
+  const size_t need = sa_hip_decode_step_workspace_bytes(kv, splits);
   if (!workspace || workspace_bytes < need)
     return fail(SA_HIP_EINVAL, "%s: workspace of %zu bytes needed, %zu given", op, need, workspace_bytes);
   if (!aligned16(workspace)) return fail(SA_HIP_EINVAL, "%s: workspace must be 16-byte aligned", op);
@@ -915,7 +901,7 @@ int sa_hip_decode_step_online(const sa_paged_kv* kv, const float* k, const float
   const char* op = "decode_step_online";
   if (!seal) return fail(SA_HIP_EINVAL, "%s: null online seal", op);
   if (!kv || kv->batch <= 0) return fail(SA_HIP_EINVAL, "%s: null sa_paged_kv or empty batch", op);
-  const size_t need = step_min_bytes(kv, splits);
+  const size_t need = sa_hip_decode_step_workspace_bytes(kv, splits);
   if (!workspace || workspace_bytes < need)
     return fail(SA_HIP_EINVAL, "%s: workspace of %zu bytes needed, %zu given", op, need, workspace_bytes);
   if (!aligned16(workspace)) return fail(SA_HIP_EINVAL, "%s: workspace must be 16-byte aligned", op);

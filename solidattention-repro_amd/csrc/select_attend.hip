@@ -1616,7 +1616,10 @@ int32_t split_step_splits(const SelectAttendLaunch& s) {
     if (!s.append || !select_attend_rows_supported(s.query_heads, s.kv_heads, s.rep_heads, s.select_groups, hd))
       return 0;
   } else if (shared) {
-    if (!select_attend_shared_supported(s.batch, s.query_heads, s.kv_heads, s.rep_heads, s.select_groups,
+    // (every workgroup reads every head's query: an output written over it
+    // would reach the workgroups that score late)
+    if (s.out == s.query ||
+        !select_attend_shared_supported(s.batch, s.query_heads, s.kv_heads, s.rep_heads, s.select_groups,
                                         s.rep_stride))
       return 0;
   } else if (group == 8) {

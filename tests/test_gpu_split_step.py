@@ -103,24 +103,3 @@ def test_split_step_without_a_page(hip, hq):
     changed = np.unique(np.nonzero((after != before).any(axis=(2, 3, 4)))[0])
     assert changed.tolist() == [int(case.table[1, 40])]
     assert int(ws[:2].abs().sum().item()) == 0
-
-
-def test_split_step_smaller_workspaces(hip):
-    """A workspace without room for the step's own records (counters, the
-    caller's records and the scores only) still serves the call."""
-    hq, hkv = 16, 8
-    case = make_case(78, 1, hq, hkv, [32 * 200 + 9])
-    rng = np.random.default_rng(6)
-    k, v = (to_dev(rng.standard_normal((1, hkv, D)).astype(np.float32)) for _ in range(2))
-    outs = []
-    for room in (True, False):
-        kv = device_kv(case)
-        ws, nbytes = hip.decode_step_workspace(kv, 2)
-        if not room:
-            records = (2 * hq * (D + 4) * 4 + 255) // 256 * 256
-            nbytes = 256 + records + hq * kv.rep_stride * 4
-        outs.append(hip.decode_step(kv, k, v, 0, to_dev(case.query), hkv, 64, 4, 8, SCALE, ws[:nbytes // 4],
-                                    splits=2))
-    torch.cuda.synchronize()
-    assert torch.equal(outs[0][0], outs[1][0]) and torch.equal(outs[0][1], outs[1][1])
-    assert_close_2e3(outs[0][2].cpu().numpy(), outs[1][2].cpu().numpy())
