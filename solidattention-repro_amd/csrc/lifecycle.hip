@@ -162,8 +162,10 @@ __global__ __launch_bounds__(kOnlineThreads) void append_seal_online_kernel(cons
   const int64_t page = table_page(p, b, pos / kPageTokens);
   int arrived = -1;
   if (arrive) {
-    // the counters are in registers before this workgroup counts as arrived
+    // every wave reads the counters for itself: all of them have them in
+    // registers before the workgroup counts as arrived
     asm volatile("" ::"s"(s0), "s"(page) : "memory");
+    __syncthreads();
     if (tid == 0) arrived = __hip_atomic_fetch_add(arrive + b, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
   const bool last = arrived == static_cast<int>(gridDim.x) - 1;  // (thread 0)
