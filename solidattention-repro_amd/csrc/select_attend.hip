@@ -172,16 +172,29 @@ __device__ inline bool append_seal_head(const Params& p, int b, int g, int64_t& 
   return true;
 }
 
-// Sequence counters of one decode step.  Every workgroup of sequence b reads
-// seq_len, sealed and generation at its start and adds 1 to arrive[b] after
-// its append; the workgroup that brings the count to kv_heads (all others
-// have read the counters by then) writes the new values and clears the count.
+// Sequence counters of one decode step.  Every wave of sequence b's workgroups
+// reads seq_len, sealed and generation at its start; behind the first barrier
+// after that a workgroup adds 1 to arrive[b].  The workgroup that brings the
+// count to kv_heads (all waves of all others have read the counters by then)
+// writes the new values and clears the count.
 struct SeqCommit {
   int gen = 0;
   int added = 0;
   int arrived = -1;
   bool appended = false;
 };
+
+// The wave's own copies of the counters are in registers from here on.
+__device__ inline void counters_read(int64_t len, int n) {
+  asm volatile("" ::"v"(static_cast<int>(len)), "v"(n) : "memory");
+}
+
+// Behind a workgroup barrier that follows every wave's counters_read().  The
+// count is used at the end of the kernel (commit_sequence()), so that its
+// round trip overlaps the scoring.
+__device__ inline void arrive_sequence(const Params& p, int b, SeqCommit& c) {
+  if (threadIdx.x == 0) c.arrived = atomicAdd(&p.arrive[b], 1);
+}
 
 __device__ inline void commit_sequence(const Params& p, int b, int64_t len, int n, const SeqCommit& c) {
   if (c.arrived != p.v.kv_heads - 1) return;
@@ -735,15 +748,14 @@ __device__ inline void decode_body(const Params& p, const Prod& qp) {
   if (have_pre) sel::score_prefetch(a, SPLIT ? tid % kHalf : tid, pre, SPLIT ? tid / kHalf * sel::kScoreBatch : 0);
 
   // ---- 1. append + seal (decode step) ---------------------------------------
-  // The arrival count is read at the end of the kernel, so that its round
-  // trip overlaps the scoring; the representatives a seal wrote are visible
-  // to the scoring after the query barrier below.
+  // The representatives a seal wrote are visible to the scoring after the
+  // query barrier below.
   SeqCommit commit{};
   if (APPEND) {
     commit.gen = p.generation ? p.generation[b] : 0;
     commit.appended = append_seal_head<G, F16, ONLINE, kProd>(p, b, g, len, n, commit.added,
                                                               reinterpret_cast<float*>(keys), tok);
-    if (!SPLIT && tid == 0) commit.arrived = atomicAdd(&p.arrive[b], 1);
+    counters_read(len, n);
   }
 
   attn::WaveState<G> st;
@@ -761,6 +773,7 @@ __device__ inline void decode_body(const Params& p, const Prod& qp) {
   } else if (n_ok && !bs.take_all) {  // (a budget that takes every block needs no scores)
     if (!kProd && tid < G * D) q_s[tid] = q_entry;
     __syncthreads();
+    if (APPEND && !SPLIT) arrive_sequence(p, b, commit);
     if constexpr (SPLIT) {
       score_halves<G, GR>(a, q_s, n, keys, reinterpret_cast<float*>(&cs), pre, have_pre);
     } else if constexpr (kPrefetch) {
@@ -768,10 +781,12 @@ __device__ inline void decode_body(const Params& p, const Prod& qp) {
     } else {
       sel::score_blocks<GR, kThreads>(a, q_s, n, keys, nullptr);
     }
+  } else if (kProd || (APPEND && !SPLIT)) {
+    __syncthreads();  // (no scoring barrier) q_s complete, the counters read
+    if (!SPLIT) arrive_sequence(p, b, commit);
   }
   if (wave == kWaves - 1) cl.early[lane] = early;
   if (tid == 0) cl.late_ready = 0;
-  if (kProd && !(n_ok && !bs.take_all)) __syncthreads();  // q_s complete (no scoring barrier)
   st.init(kProd ? q_s : q_group, p.qscale, lg.col);
   // the walk's view of the sequence (a length below the sealed blocks is
   // flagged and walked as no tail)
@@ -947,7 +962,7 @@ __global__ __launch_bounds__(kThreads) void decode_kernel_shared(const Params p)
   if (APPEND) {
     commit.gen = p.generation ? p.generation[b] : 0;
     commit.appended = append_seal_shared<F16>(p, b, g, len, n, commit.added);
-    if (!SPLIT && tid == 0) commit.arrived = atomicAdd(&p.arrive[b], 1);
+    counters_read(len, n);
   }
 
   attn::WaveState<G> st;
@@ -973,6 +988,7 @@ __global__ __launch_bounds__(kThreads) void decode_kernel_shared(const Params p)
     a.rep_stride = p.rep_stride;
     sel::load_query_t<kThreads>(a, q_t);
     __syncthreads();  // the query, and the representatives this workgroup sealed
+    if (APPEND && !SPLIT) arrive_sequence(p, b, commit);
     const int hps = p.query_heads;
     const float heads_f = static_cast<float>(hps);
     // dot / heads for a power-of-two head count: the product with the exact
@@ -1002,6 +1018,9 @@ __global__ __launch_bounds__(kThreads) void decode_kernel_shared(const Params p)
       }
       __syncthreads();
     }
+  } else if (APPEND && !SPLIT) {
+    __syncthreads();  // (no scoring barrier)
+    arrive_sequence(p, b, commit);
   }
   if (wave == kWaves - 1) cl.early[lane] = early;
   if (tid == 0) cl.late_ready = 0;
@@ -1193,8 +1212,8 @@ __global__ __launch_bounds__(kThreads, G == 4 && LPR > 8 ? 2 : 4) void decode_ke
   if (APPEND) {
     commit.gen = p.generation ? p.generation[b] : 0;
     commit.appended = append_seal_head_any<F16>(p, b, g, hd, len, n, commit.added);
+    counters_read(len, n);
   }
-  if (!SPLIT && tid == 0) commit.arrived = atomicAdd(&p.arrive[b], 1);
 
   State st;
   st.init(q_group, hd, p.qscale, lane);
@@ -1206,7 +1225,8 @@ __global__ __launch_bounds__(kThreads, G == 4 && LPR > 8 ? 2 : 4) void decode_ke
            : sel::Budget{0, 0, 0, false, true};
   const Forced fb = forced_blocks(bs, n);
   const int32_t early = wave == kWaves - 1 ? early_page(p, b, n, fb, lane) : -1;
-  __syncthreads();  // the query rows, and the representatives this workgroup sealed
+  __syncthreads();  // the query rows, the representatives this workgroup sealed, the counters read
+  if (!SPLIT) arrive_sequence(p, b, commit);
   if (SPLIT && p.scores) {
     if (n_ok && !bs.take_all) keys_from_scores(p, out_row, n, keys);
   } else if (n_ok && !bs.take_all) {  // (a budget that takes every block needs no scores)
@@ -1350,7 +1370,7 @@ __global__ __launch_bounds__(kThreads) void decode_kernel_staged(const Params p)
   int64_t len = p.seq_len[b];
   int n = p.sealed[b];
 
-  // ---- 1. append + seal (decode step; arrival read at the end, as above) ------
+  // ---- 1. append + seal (decode step) -----------------------------------------
   // A step that seals a block appends and seals here, before the scoring.
   // Otherwise nothing reads the new token before the page walk: wave 0
   // stores it at the start of the walk phase, before it lists the tail (the
@@ -1370,7 +1390,7 @@ __global__ __launch_bounds__(kThreads) void decode_kernel_staged(const Params p)
       tail_page = table_page(p.v, b, len / kPageTokens);
       if (wave == 0) token = token_quad<F16>(p, b, g, lane);
     }
-    if (!SPLIT && tid == 0) commit.arrived = atomicAdd(&p.arrive[b], 1);
+    counters_read(len, n);
   }
 
   attn::WaveState<G> st;
@@ -1401,6 +1421,7 @@ __global__ __launch_bounds__(kThreads) void decode_kernel_staged(const Params p)
 #pragma unroll
     for (int i = 0; i < kQLoads; ++i) q_t[(tid % D) * G + tid / D + i * (kThreads / D)] = q_entry[i];
     __syncthreads();
+    if (APPEND && !SPLIT) arrive_sequence(p, b, commit);
     // one block per lane up to 512 blocks (two per lane would leave waves
     // without blocks), else two
     if (n <= kThreads) {
@@ -1408,6 +1429,9 @@ __global__ __launch_bounds__(kThreads) void decode_kernel_staged(const Params p)
     } else {
       sel::score_blocks_vec<GR, 2, kThreads>(a, q_t, n, keys, nullptr, tid);
     }
+  } else if (APPEND && !SPLIT) {
+    __syncthreads();  // (no scoring barrier)
+    arrive_sequence(p, b, commit);
   }
   if (ONLINE && deferred && tail_page >= 0) {
     // the group's query rows of this step to the ring (read by later seals)

@@ -79,7 +79,7 @@ def reached_without_barrier(code):
     return bad
 
 
-@pytest.mark.parametrize("family", ["append_seal_online_kernel"])
+@pytest.mark.parametrize("family", ["append_seal_online_kernel", "decode_kernel"])
 def test_arrival_behind_a_barrier(kernels, family):
     members = {n: c for n, c in kernels.items() if family in n and any(is_arrival(i[1], i[2]) for i in c)}
     assert members, family
