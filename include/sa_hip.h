@@ -312,8 +312,13 @@ int sa_hip_select_attend(const sa_paged_kv* kv, const float* query,
 
 /* ---- R8/R9/R4 + R3 + R6 fused: one layer's whole decode step ------------- */
 
-/* Workspace of sa_hip_decode_step: `batch` int32 arrival counters (padded
- * to 256 bytes) followed by the attention's split records (padded to 256
+#define SA_HIP_STEP_COUNTER_BYTES (256u << 10)
+
+/* Workspace of sa_hip_decode_step: SA_HIP_STEP_COUNTER_BYTES of int32
+ * arrival counters (one per sequence, room for 65536 whatever the batch, so
+ * that calls of different batches may share a workspace: none of them writes
+ * anything else over another's counters) followed by the attention's split
+ * records (padded to 256
  * bytes) and the split selection's scores (batch x query_heads x rep_stride
  * floats; used when the step runs as separate launches with few lists, and
  * at every head_dim other than 128), and at least as large as the counters

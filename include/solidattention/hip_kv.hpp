@@ -239,7 +239,7 @@ class SparseDecoder {
                      hipStream_t stream = nullptr, int32_t* status = nullptr) {
     const sa_paged_kv kv = pool.view();
     // the split records of the non-fused path sit after the arrival counters
-    const std::size_t skip = arrive_bytes(pool.batch());
+    const std::size_t skip = SA_HIP_STEP_COUNTER_BYTES;
     check(sa_hip_select_attend(&kv, query, &params_, scale, selected_.get(), counts_.get(), out,
                                step_workspace_.get() + skip / 4, step_workspace_bytes_ - skip, step_splits_, status,
                                stream),
@@ -314,9 +314,6 @@ class SparseDecoder {
     const sa_paged_kv kv = pool.view();
     return sa_hip_decode_step_workspace_bytes(&kv, splits);
   }
-  // the decode-step workspace starts with one int32 arrival counter per
-  // sequence, padded to 256 bytes (sa_hip_decode_step_workspace_bytes)
-  static std::size_t arrive_bytes(std::size_t batch) { return (batch * 4 + 255) / 256 * 256; }
 };
 
 struct Correction {

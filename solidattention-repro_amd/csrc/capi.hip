@@ -635,9 +635,14 @@ int sa_hip_select_attend(const sa_paged_kv* kv, const float* query, const sa_sel
   return check_hip(sa::launch_select_attend(f, as_stream(stream)), "select_attend launch");
 }
 
-// Decode-step workspace: [batch] int32 arrival counters (padded to 256 B),
-// then the attention's split records when the step is not fused.
-static size_t arrive_bytes(int32_t batch) { return (static_cast<size_t>(batch) * 4 + 255) / 256 * 256; }
+// Decode-step workspace: the arrival counters, then the attention's split
+// records when the step is not fused.  The counters' share does not depend on
+// the batch: with records right behind a small batch's counters they would lie
+// over those of a larger batch's further sequences, which a step on the same
+// workspace expects to find at zero.
+static size_t arrive_bytes(int32_t batch) {
+  return std::max<size_t>(SA_HIP_STEP_COUNTER_BYTES, (static_cast<size_t>(batch) * 4 + 255) / 256 * 256);
+}
 
 // When the step runs as separate launches its split selection (the only
 // scoring at a head_dim other than 128; at 128 the shared selection's, for
@@ -653,7 +658,6 @@ static size_t split_scores_bytes(const sa_paged_kv* kv, int32_t select_groups) {
 }
 
 // Records of the step with several workgroups per list.
-
 static size_t split_step_bytes(const sa_paged_kv* kv, int32_t splits) {
   const size_t records =
       static_cast<size_t>(kv->batch) * kv->query_heads * splits * sa::part_stride(kv->head_dim) * sizeof(float);

@@ -505,8 +505,12 @@ def select_attend(kv: PagedKV, query, select_groups, budget, init, local, scale,
     return selected, counts, out
 
 
+STEP_COUNTER_BYTES = 256 << 10  # of a decode-step workspace: the arrival counters, room for any batch
+
+
 def decode_step_workspace(kv: PagedKV, splits=1, device="cuda"):
-    """Zeroed workspace for decode_step (arrival counters + split records)."""
+    """Zeroed workspace for decode_step (arrival counters + split records);
+    steps of different batches may share one, one after the other."""
     import torch
     n = lib().sa_hip_decode_step_workspace_bytes(C.byref(kv.struct()), splits)
     return torch.zeros(max(n // 4, 1), dtype=torch.int32, device=device), n
