@@ -315,17 +315,16 @@ int sa_hip_select_attend(const sa_paged_kv* kv, const float* query,
 #define SA_HIP_STEP_COUNTER_BYTES (256u << 10)
 
 /* Workspace of sa_hip_decode_step: SA_HIP_STEP_COUNTER_BYTES of int32
- * arrival counters (one per sequence, room for 65536 whatever the batch, so
- * that calls of different batches may share a workspace: none of them writes
- * anything else over another's counters) followed by the attention's split
- * records (padded to 256
- * bytes) and the split selection's scores (batch x query_heads x rep_stride
- * floats; used when the step runs as separate launches with few lists, and
- * at every head_dim other than 128), and at least as large as the counters
- * and the partial records of a one-launch step that spreads each list over
- * several workgroups.  The caller
- * zeroes it ONCE before the first call; every call leaves the counters at
- * zero again.  Calls sharing a workspace must not run concurrently. */
+ * arrival counters (one per sequence, room for 65536 whatever the batch),
+ * then partial records (the attention's splits, or those of a one-launch step
+ * that spreads each list over several workgroups; padded to 256 bytes) and
+ * the split selection's scores (batch x query_heads x rep_stride floats; used
+ * when the step runs as separate launches with few lists, and at every
+ * head_dim other than 128).  The size grows with the batch, query_heads,
+ * head_dim, rep_stride and splits: one workspace serves every step up to the
+ * one it was sized for.  The caller zeroes it ONCE before the first call;
+ * every call leaves the counters at zero again and writes nothing else over
+ * them.  Calls sharing a workspace must not run concurrently. */
 size_t sa_hip_decode_step_workspace_bytes(const sa_paged_kv* kv,
                                           int32_t splits);
 

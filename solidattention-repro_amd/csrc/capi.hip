@@ -664,14 +664,19 @@ static size_t split_step_bytes(const sa_paged_kv* kv, int32_t splits) {
   return (records + 255) / 256 * 256;
 }
 
+// Grows with the batch, the query heads, the head_dim, rep_stride and splits
+// (and does not depend on the KV heads), so that a workspace sized for a
+// program's largest step serves its smaller ones, although some of those
+// spread each list over more workgroups.
 size_t sa_hip_decode_step_workspace_bytes(const sa_paged_kv* kv, int32_t splits) {
   if (!kv || kv->batch <= 0) return 0;
-  const size_t need =
-      arrive_bytes(kv->batch) + split_records_bytes(kv, splits) + split_scores_bytes(kv, kv->query_heads);
-  if (kv->kv_heads <= 0 || kv->query_heads <= 0 || kv->head_dim <= 0) return need;
-  const int32_t cap = sa::split_step_cap(kv->batch, kv->query_heads, kv->kv_heads, kv->head_dim);
-  return std::max(need,
-                  arrive_bytes(kv->batch) + split_step_bytes(kv, cap) + split_scores_bytes(kv, kv->query_heads));
+  const size_t counters_and_scores = arrive_bytes(kv->batch) + split_scores_bytes(kv, kv->query_heads);
+  const size_t records = split_records_bytes(kv, splits);
+  if (kv->kv_heads <= 0 || kv->query_heads <= 0 || kv->head_dim <= 0) return counters_and_scores + records;
+  const size_t step_records =
+      static_cast<size_t>(sa::split_step_records(kv->batch, kv->query_heads)) * sa::part_stride(kv->head_dim) *
+      sizeof(float);
+  return counters_and_scores + std::max(records, (step_records + 255) / 256 * 256);
 }
 
 // Whether the step after append + seal runs as a scoring launch and a launch of

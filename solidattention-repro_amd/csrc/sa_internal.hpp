@@ -204,10 +204,11 @@ bool select_attend_supported(int32_t query_heads, int32_t kv_heads, int32_t sele
 int select_attend_per_cu(int32_t query_heads, int32_t kv_heads);
 // The step with several workgroups per (sequence, KV head), for fewer lists
 // than the device has workgroup slots; one launch whose last workgroups merge
-// the partial records (query_heads / kv_heads * part_stride(head_dim) floats
-// per workgroup).  cap: the most splits any call of this geometry uses (sizes
-// the workspace); splits: this call's, 0 where the step does not apply.
-int32_t split_step_cap(int32_t batch, int32_t query_heads, int32_t kv_heads, int32_t head_dim);
+// the partial records (part_stride(head_dim) floats per query head and
+// workgroup).  records: at least as many as any step of up to `batch`
+// sequences and query_heads query heads writes (sizes the workspace); splits:
+// this call's per list, 0 where the step does not apply.
+int64_t split_step_records(int32_t batch, int32_t query_heads);
 int32_t split_step_splits(const SelectAttendLaunch& s);
 // s.append 0: the token is already appended and sealed.  s.arrive as for the
 // one-launch step.

@@ -1611,16 +1611,28 @@ static int split_field_bits(int32_t kv_heads) {
   return bits > 8 ? 8 : bits;
 }
 
-int32_t split_step_cap(int32_t batch, int32_t query_heads, int32_t kv_heads, int32_t head_dim) {
+// Workgroups the device holds at once, and the query heads' records they make.
+static int64_t split_slots(int32_t query_heads, int32_t kv_heads, int32_t head_dim) {
+  return (head_dim == kHeadDim && query_heads / kv_heads >= 4 ? 1 : 2) * static_cast<int64_t>(compute_units());
+}
+constexpr int kSlotRecords = 8;  // per compute unit, at most: 8 heads of one workgroup, or 4 of each of two
+
+// The most splits of a list any call of this geometry uses.
+static int32_t split_step_cap(int32_t batch, int32_t query_heads, int32_t kv_heads, int32_t head_dim) {
   if (batch <= 0 || kv_heads <= 0) return 1;
   const int bits = split_field_bits(kv_heads);
   if (bits < 1) return 1;
-  const int64_t lists = static_cast<int64_t>(batch) * kv_heads;
-  const int64_t slots =
-      (head_dim == kHeadDim && query_heads / kv_heads >= 4 ? 1 : 2) * static_cast<int64_t>(compute_units());
   const int64_t most = (int64_t{1} << bits) - 1 < kMaxStepSplits ? (int64_t{1} << bits) - 1 : kMaxStepSplits;
-  const int64_t want = slots / lists;
+  const int64_t want = split_slots(query_heads, kv_heads, head_dim) / (static_cast<int64_t>(batch) * kv_heads);
   return static_cast<int32_t>(want < 1 ? 1 : (want < most ? want : most));
+}
+
+int64_t split_step_records(int32_t batch, int32_t query_heads) {
+  const int64_t heads = static_cast<int64_t>(batch) * query_heads;  // one split each
+  const int64_t held = kSlotRecords * static_cast<int64_t>(compute_units());
+  const int64_t most = heads * kMaxStepSplits;
+  const int64_t split = most < held ? most : held;
+  return heads > split ? heads : split;
 }
 
 int32_t split_step_splits(const SelectAttendLaunch& s) {

@@ -89,3 +89,46 @@ def test_one_workspace_over_batches(hip, first):
         for a, e in zip(got, own):
             assert torch.equal(a, e), second
         assert int(ws[:sa.STEP_COUNTER_BYTES // 4].abs().sum().item()) == 0
+
+
+HEADS = [(16, 8), (8, 8), (32, 8), (64, 8), (16, 4), (8, 1), (20, 20), (32, 32), (3, 3)]
+
+
+@pytest.mark.parametrize("hq,hkv", HEADS)
+@pytest.mark.parametrize("head_dim", [128, 64, 256])
+@pytest.mark.parametrize("splits", [1, 2, 16])
+def test_size_serves_every_smaller_batch(hq, hkv, head_dim, splits):
+    sizes = [nbytes(b, hq, hkv, splits, head_dim=head_dim) for b in range(1, 300)]
+    assert sizes == sorted(sizes)
+
+
+@pytest.mark.parametrize("batch", [1, 7, 33, 64, 500])
+def test_size_serves_every_smaller_geometry(batch):
+    """... and no fewer heads, shorter rows or fewer splits ask for more."""
+    for d in (64, 128, 256):
+        for splits in (1, 4):
+            sizes = [nbytes(batch, hq, hkv, splits, head_dim=d) for hq, hkv in sorted(HEADS)]
+            assert sizes == sorted(sizes), (d, splits)
+            assert nbytes(batch, 16, 8, splits, head_dim=d) == nbytes(batch, 16, 4, splits, head_dim=d)
+    assert nbytes(batch, 16, 8, 1) <= nbytes(batch, 16, 8, 2) <= nbytes(batch, 16, 8, 16)
+    assert nbytes(batch, 16, 8, head_dim=64) <= nbytes(batch, 16, 8) <= nbytes(batch, 16, 8, head_dim=256)
+    assert nbytes(batch, 16, 8, rep_stride=32) <= nbytes(batch, 16, 8)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("form", list(FORMS))
+@pytest.mark.parametrize("batch", [1, 2, 8, 33])
+def test_workspace_of_a_larger_batch(hip, form, batch):
+    """A workspace of the size of 40 sequences' step serves smaller steps,
+    none of which writes past its end or leaves a counter set."""
+    hq, hkv, d, splits, _, online = FORMS[form]
+    big, _ = random_kv(40, hq, hkv, d, 40, hq if online else hkv, 1)
+    size = sa.decode_step_workspace(big, splits)[1] // 4
+    ws = torch.zeros(size + 4096, dtype=torch.int32, device="cuda")
+    ws[size:] = 7
+    got, kv = run(form, batch, ws[:size], 5)
+    own, _ = run(form, batch, sa.decode_step_workspace(kv, splits)[0], 5)
+    for a, e in zip(got, own):
+        assert torch.equal(a, e)
+    assert int(ws[:sa.STEP_COUNTER_BYTES // 4].abs().sum().item()) == 0
+    assert bool((ws[size:] == 7).all())
