@@ -787,7 +787,8 @@ static int decode_step_run(const sa_paged_kv* kv, const float* k, const float* v
       sa::decode_step_qkv_supported(kv->query_heads, kv->kv_heads, params->select_groups, kv->head_dim)) {
     // the producer's partial launch, then several workgroups per list that run
     // its epilogue
-    const sa::SelectAttendLaunch f = step_launch();
+    sa::SelectAttendLaunch f = step_launch();
+    f.writes_query = true;
     const int32_t s = sa::split_step_splits(f);
     if (s >= 1) {
       sa::qkv::ReduceParams r;

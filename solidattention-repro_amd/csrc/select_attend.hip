@@ -1635,11 +1635,34 @@ int64_t split_step_records(int32_t batch, int32_t query_heads) {
   return heads > split ? heads : split;
 }
 
+// Whether the last workgroup of a list may write its output rows while other
+// lists' workgroups still read the step's inputs.  Where the output is the
+// query's own buffer those rows hold the list's own queries, which all of its
+// workgroups have read; not so where every workgroup reads every head's query
+// (the shared selection), nor where each workgroup writes its queries itself
+// (a list's workgroups may run on XCDs with L2s of their own, and a query
+// would reach memory after the output).
+static bool out_apart(const SelectAttendLaunch& s, int hd, bool all_queries) {
+  const size_t row = static_cast<size_t>(s.batch) * hd;
+  const uintptr_t out = reinterpret_cast<uintptr_t>(s.out);
+  const uintptr_t end = out + row * s.query_heads * sizeof(float);
+  auto apart = [&](const void* x, size_t bytes) {
+    const uintptr_t at = reinterpret_cast<uintptr_t>(x);
+    return !x || at >= end || at + bytes <= out;
+  };
+  const size_t token = row * s.kv_heads;
+  if (s.append && !(apart(s.k, token * 4) && apart(s.v, token * 4) && apart(s.k16, token * 2) &&
+                    apart(s.v16, token * 2)))
+    return false;
+  return apart(s.query, end - out) || (s.out == s.query && !all_queries && !s.writes_query);
+}
+
 int32_t split_step_splits(const SelectAttendLaunch& s) {
   if (s.ring || s.kv_heads <= 0 || split_field_bits(s.kv_heads) < 1) return 0;
   const int hd = s.head_dim > 0 ? s.head_dim : kHeadDim;
   const int group = s.query_heads / s.kv_heads;
   const bool shared = s.select_groups != s.kv_heads;
+  if (!out_apart(s, hd, shared && !s.scores)) return 0;
   if (s.scores) {
     if (s.append || s.select_groups <= 0 || s.kv_heads % s.select_groups != 0) return 0;
     if (hd != kHeadDim ? hd > rows::kMaxHeadDim || hd % 8 != 0 || (group != 1 && group != 2 && group != 4)
@@ -1652,10 +1675,7 @@ int32_t split_step_splits(const SelectAttendLaunch& s) {
     if (!s.append || !select_attend_rows_supported(s.query_heads, s.kv_heads, s.rep_heads, s.select_groups, hd))
       return 0;
   } else if (shared) {
-    // (every workgroup reads every head's query: an output written over it
-    // would reach the workgroups that score late)
-    if (s.out == s.query ||
-        !select_attend_shared_supported(s.batch, s.query_heads, s.kv_heads, s.rep_heads, s.select_groups,
+    if (!select_attend_shared_supported(s.batch, s.query_heads, s.kv_heads, s.rep_heads, s.select_groups,
                                         s.rep_stride))
       return 0;
   } else if (group == 8) {
