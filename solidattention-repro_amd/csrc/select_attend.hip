@@ -583,15 +583,12 @@ struct PlanPages {
   }
 };
 
-// G = query heads per KV head; GR = query heads sharing one representative
-// row (G for per-KV-head representatives, 1 for per-query-head ones);
-// APPEND: decode step (append + seal first); F16: raw FP16 K/V input.
 // Scores with every lane of the workgroup loading, 256 blocks at a time: lanes
 // tid and tid + 256 share a block.  With one representative row (GR == G) each
 // takes 64 of its 128 values, all in flight at once, and the first lane's
-// partial dots are handed to the second, which goes on with the sum (while the
-// first loads the next 256 blocks); with a row per query head (G = 2) each
-// takes a row.  The reference's operations in its order, as sel::score_one().
+// partial dots are handed to the second, which goes on with the sum behind the
+// barrier (while the first loads the next 256 blocks); with a row per query
+// head (G = 2) each takes a row.  The reference's operations in its order, as sel::score_one().
 // part: 2 G * 256 floats of LDS.  One lane per block leaves half the waves
 // idle up to 256 blocks and takes two or more round trips to memory.
 template <int G, int GR>
@@ -601,7 +598,6 @@ __device__ inline void score_halves(const sel::ScoreArgs& a, const float* q_s, i
   constexpr int kB = sel::kScoreBatch;
   static_assert(D == 2 * kB, "two batches per representative row");
   static_assert(GR == G || (G == 2 && GR == 1), "one row, or a half of the lanes per row");
-  const int half = threadIdx.x / kHalf;  // wave-uniform
   const float heads_f = static_cast<float>(a.heads_per_sel);
   int qoff = 0;
   asm volatile("" : "+s"(qoff));
@@ -626,24 +622,25 @@ __device__ inline void score_halves(const sel::ScoreArgs& a, const float* q_s, i
       float dot[G];
 #pragma unroll
       for (int j = 0; j < G; ++j) dot[j] = 0.0f;
+      const int half = __builtin_amdgcn_readfirstlane(threadIdx.x / kHalf);  // of whole waves
       if (valid && !(have_pre && c0 == 0)) sel::score_prefetch(row, blk, pre, half * kB);
-      if (half == 1) {
-        __syncthreads();
-#pragma unroll
-        for (int j = 0; j < G; ++j) dot[j] = part_c[j * kHalf];
-      }
-      if (valid) sum(dot, 0, half * kB);
       if (half == 0) {
+        if (valid) sum(dot, 0, 0);
 #pragma unroll
         for (int j = 0; j < G; ++j) part_c[j * kHalf] = dot[j];
-        __syncthreads();
-      } else if (valid) {
+      }
+      __syncthreads();
+      if (half == 1 && valid) {
+#pragma unroll
+        for (int j = 0; j < G; ++j) dot[j] = part_c[j * kHalf];
+        sum(dot, 0, kB);
         float score = 0.0f;
 #pragma unroll
         for (int j = 0; j < G; ++j) score = score + dot[j] / heads_f;
         keys[blk] = sel::order_key(score);
       }
     } else {
+      const int half = threadIdx.x / kHalf;
       if (valid) {
         row.h_first = a.h_first + half;
         float dot[1] = {0.0f};
@@ -668,6 +665,9 @@ __device__ inline void score_halves(const sel::ScoreArgs& a, const float* q_s, i
 // No q/k/v producer: the step's query and token are inputs.
 struct NoProducer {};
 
+// G = query heads per KV head; GR = query heads sharing one representative
+// row (G for per-KV-head representatives, 1 for per-query-head ones);
+// APPEND: decode step (append + seal first); F16: raw FP16 K/V input.
 // Prod = qkv::ReduceParams: the step takes the q/k/v projection's K-slice
 // partials instead of q, k and v, and runs their epilogue (qkv_epilogue.hpp)
 // for its own heads at entry: wave 0 the group's query heads (32 lanes each),

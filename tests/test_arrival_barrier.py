@@ -85,3 +85,25 @@ def test_arrival_behind_a_barrier(kernels, family):
     assert members, family
     bad = {n: b for n, b in ((n, reached_without_barrier(c)) for n, c in members.items()) if b}
     assert not bad, f"arrivals reached without a barrier: {bad}"
+
+
+def masked_barriers(code):
+    """The addresses of barriers behind a narrowing of the lane mask that is not undone before them."""
+    bad, narrowed = [], False
+    for address, mnemonic, operands, _ in code:
+        if "_saveexec_" in mnemonic:
+            narrowed = True
+        elif operands.strip().startswith("exec,") or mnemonic == "s_branch":  # undone, or another path's code follows
+            narrowed = False
+        elif mnemonic == "s_barrier" and narrowed:
+            bad.append(hex(address))
+    return bad
+
+
+def test_every_lane_reaches_the_same_barriers(kernels):
+    """A workgroup barrier stands in code that all of the workgroup's waves
+    run, not in the branch of some of its lanes (two halves of a workgroup at
+    two barriers only pair up for as long as the compiler keeps each branch's
+    skip)."""
+    bad = {n: b for n, b in ((n, masked_barriers(c)) for n, c in kernels.items()) if b}
+    assert not bad, f"barriers under a lane mask: {bad}"
