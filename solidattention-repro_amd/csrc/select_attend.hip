@@ -261,10 +261,14 @@ __device__ inline void store_record(float* rec, int d, float mx, float lw, float
   store_agent(rec + kPartPad + d, aw);
 }
 
+// The most workgroups of a list: their 128 waves are two walkers per lane of the
+// plan (PlanPages::plan_late_split()).  One sequence, 16/8 heads, 16K tokens,
+// budget 128: at most 4 workgroups 33.1 us, 8: 26.3, 16: 25.2.
+constexpr int kMaxStepSplits = 16;
+
 // The list's records merged (log-sum-exp, in split order) into its G output
 // rows of hd values; the loads of all records of a batch are in flight
 // together.
-constexpr int kMaxStepSplits = 16;
 
 template <int G>
 __device__ inline void merge_split_records(const Params& p, int b, int g, int hd) {
@@ -494,8 +498,9 @@ struct PlanPages {
   // The split plan: walker u = wave * splits + z of 8 * splits (<= 128), the
   // selecting waves first.  No wave has a late position before its
   // workgroup's selection is done, so a walker starts on them after the
-  // larger of its forced positions and the selection (kSelectPages), and the
-  // ranges even out the sums.  Each lane plans two walkers; a prefix sum gives
+  // larger of its forced positions and the selection (kSelectPages; counted as
+  // 1 to 3 pages the step takes the same time to 2%, as none up to 4% more), and
+  // the ranges even out the sums.  Each lane plans two walkers; a prefix sum gives
   // where a walker's range begins.
   __device__ inline int split_want(int u, int late_n) const {
     const int walkers = kWaves * splits;
@@ -1602,7 +1607,10 @@ hipError_t launch_shared(const Params& p, int batch, hipStream_t stream) {
 
 // ---- the step with several workgroups per list ----------------------------------
 // Every workgroup of a list scores all of it; longer lists, and groups of
-// several KV heads, take their scores from a scoring launch (s.scores).
+// several KV heads, take their scores from a scoring launch (s.scores).  Budget
+// 64, 16, 32 or 64 query heads on 8 KV heads: at 500 blocks the two are within
+// 1%; at 1000 scoring for itself costs 3 to 6% with 2 or 4 sequences and saves 5%
+// with 16 (4 and 8 heads per KV head; 12% more at 2); at 1450 it costs 40 to 54%.
 constexpr int kMaxSplitStepBlocks = 1024;
 
 // Bits of a KV head's field in a sequence's 32-bit arrival counter.
@@ -1611,19 +1619,29 @@ static int split_field_bits(int32_t kv_heads) {
   return bits > 8 ? 8 : bits;
 }
 
-// Workgroups the device holds at once, and the query heads' records they make.
-static int64_t split_slots(int32_t query_heads, int32_t kv_heads, int32_t head_dim) {
-  return (head_dim == kHeadDim && query_heads / kv_heads >= 4 ? 1 : 2) * static_cast<int64_t>(compute_units());
+// Workgroups of 8 waves the device holds at once: one per compute unit where
+// the kernel's registers or page slots allow no more (4 and 8 query heads per
+// KV head; at another head_dim 4 heads with 16 or 32 lanes per row; the shared
+// selection's own scoring), else two.  Twice as many run in two rounds, each
+// of which scores the whole list again: 4 heads of 256, 8K tokens, 8 sequences
+// 54 us with a round's worth and 79 with two, 16 sequences 77 and 101, 24: 118
+// and 139; of 96: 31 and 45, 42 and 54, 59 and 71; shared selection of 40
+// blocks, 10 sequences of 2K tokens: 25 and 37 (8 query heads), 28 and 40 (16).
+static int64_t split_slots(int32_t query_heads, int32_t kv_heads, int32_t head_dim, bool shared) {
+  const int32_t group = query_heads / kv_heads;
+  const bool one = shared || (head_dim == kHeadDim ? group >= 4 : group >= 4 && rows::lanes_per_row(head_dim) > 8);
+  return (one ? 1 : 2) * static_cast<int64_t>(compute_units());
 }
-constexpr int kSlotRecords = 8;  // per compute unit, at most: 8 heads of one workgroup, or 4 of each of two
+constexpr int kSlotRecords = 8;  // query heads' records per compute unit, at most: 8 heads of one workgroup, or
+                                 // 4 of each of two
 
 // The most splits of a list any call of this geometry uses.
-static int32_t split_step_cap(int32_t batch, int32_t query_heads, int32_t kv_heads, int32_t head_dim) {
+static int32_t split_step_cap(int32_t batch, int32_t query_heads, int32_t kv_heads, int32_t head_dim, bool shared) {
   if (batch <= 0 || kv_heads <= 0) return 1;
   const int bits = split_field_bits(kv_heads);
   if (bits < 1) return 1;
   const int64_t most = (int64_t{1} << bits) - 1 < kMaxStepSplits ? (int64_t{1} << bits) - 1 : kMaxStepSplits;
-  const int64_t want = split_slots(query_heads, kv_heads, head_dim) / (static_cast<int64_t>(batch) * kv_heads);
+  const int64_t want = split_slots(query_heads, kv_heads, head_dim, shared) / (static_cast<int64_t>(batch) * kv_heads);
   return static_cast<int32_t>(want < 1 ? 1 : (want < most ? want : most));
 }
 
@@ -1684,7 +1702,7 @@ int32_t split_step_splits(const SelectAttendLaunch& s) {
                                       s.rep_stride)) {
     return 0;
   }
-  const int32_t cap = split_step_cap(s.batch, s.query_heads, s.kv_heads, hd);
+  const int32_t cap = split_step_cap(s.batch, s.query_heads, s.kv_heads, hd, shared && !s.scores);
   const int32_t pages = s.budget + 1;  // (a partial tail page)
   const int32_t by_pages = pages / kWaves < 1 ? 1 : pages / kWaves;
   return cap < by_pages ? cap : by_pages;
