@@ -749,6 +749,7 @@ static int decode_step_run(const sa_paged_kv* kv, const float* k, const float* v
     f.k16 = k16;
     f.v16 = v16;
     f.arrive = arrive;
+    f.launch_splits = splits;
     return f;
   };
   if (sa::general_head_dim(kv->head_dim) && (seal || !sa_hip_select_attend_fused(kv, params, splits))) {

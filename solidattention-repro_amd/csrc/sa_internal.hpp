@@ -194,6 +194,7 @@ struct SelectAttendLaunch {
   // launch_split_step, append 0: the lists' scores ([batch][select_groups]
   // [rep_stride]) from launch_scores()
   const float* scores;
+  int32_t launch_splits;  // of the separate launches this step would otherwise run as
   bool writes_query;  // fed by the q/k/v projection's partials: query, k and v are written
 };
 

@@ -1675,6 +1675,36 @@ static bool out_apart(const SelectAttendLaunch& s, int hd, bool all_queries) {
   return apart(s.query, end - out) || (s.out == s.query && !all_queries && !s.writes_query);
 }
 
+// Whether `splits` workgroups per list are better than the separate launches
+// with s.launch_splits.  They save 10 to 15 us of launches, but the arrival
+// counter's field (3 at 11 to 16 KV heads, 1 at 17 to 32), kMaxStepSplits or
+// the device's slots may allow fewer workgroups than those launches have, and
+// then each wave walks more pages.  Per layer, the launches and the split form:
+//   * up to half as many workgroups as compute units, a wave's pages decide. 4.3
+//     a wave: 42.0 and 43.4 us (16/8 heads, budget 512), 47.4 and 46.6 (32/8),
+//     59.2 and 55.8 (32/4); 5.4: 36.8 and 38.6 (16/16); 7: 61.5 and 65.0 (8/1); 8:
+//     38.1 and 45.3 (32/32); 17: 73.9 and 99.8 (16/8, 128K); 64: 63 and 199;
+//   * more than a compute unit each but less than 11 for 8 of them: the units with
+//     two workgroups are the launch's time.  10.7 pages a wave: 88.2 and 105.1 (6
+//     sequences, 16/16); 12: 115.6 and 117.7, 114.7 and 113.9 (33 and 34
+//     sequences on 8 KV heads); 16: 144.7 and 149.7, head_dim 64 88.4 and 94.4, 256
+//     259.8 and 290.1; 32: 261 and 284 (40 sequences).  Only with up to 2 query
+//     heads per KV head: of 8 (36 sequences) 208 and 197;
+//   * between and beyond, the split form: 150 workgroups 64.6 and 53.0 (8 sequences,
+//     20/20), 176 85.7 and 65.2 (64/8), 352 66.3 and 56.0 (22, 16/8).
+static bool split_step_pays(const SelectAttendLaunch& s, int32_t splits, int32_t pages) {
+  if (splits > s.launch_splits) return true;
+  const int64_t cus = compute_units();
+  const int64_t workgroups = static_cast<int64_t>(s.batch) * s.kv_heads * splits;
+  const int64_t waves = static_cast<int64_t>(kWaves) * splits;
+  if (workgroups * 2 <= cus) return pages <= 5 * waves;
+  if (workgroups > cus && workgroups * 8 < cus * 11 && s.query_heads <= 2 * s.kv_heads) {
+    const bool by_field = splits == (1 << split_field_bits(s.kv_heads)) - 1;
+    return 2 * static_cast<int64_t>(pages) <= (by_field ? 20 : 25) * waves;
+  }
+  return true;
+}
+
 int32_t split_step_splits(const SelectAttendLaunch& s) {
   if (s.ring || s.kv_heads <= 0 || split_field_bits(s.kv_heads) < 1) return 0;
   const int hd = s.head_dim > 0 ? s.head_dim : kHeadDim;
@@ -1705,7 +1735,8 @@ int32_t split_step_splits(const SelectAttendLaunch& s) {
   const int32_t cap = split_step_cap(s.batch, s.query_heads, s.kv_heads, hd, shared && !s.scores);
   const int32_t pages = s.budget + 1;  // (a partial tail page)
   const int32_t by_pages = pages / kWaves < 1 ? 1 : pages / kWaves;
-  return cap < by_pages ? cap : by_pages;
+  const int32_t splits = cap < by_pages ? cap : by_pages;
+  return split_step_pays(s, splits, pages) ? splits : 0;
 }
 
 template <bool APPEND, bool F16>
