@@ -1147,9 +1147,9 @@ __device__ inline bool append_seal_head_any(const Params& p, int b, int g, int h
 
 // Score of block blk for the group's G heads (one representative row),
 // q_s = the G query rows of hd floats in LDS.
-template <int G>
+// kBatch: its values in flight at once.
+template <int G, int kBatch>
 __device__ inline float score_block_any(const Params& p, const float* q_s, int b, int g, int hd, int blk) {
-  constexpr int kBatch = 64;  // (a whole row at head_dim 64: one round trip to memory)
   constexpr int kStep = 8;    // head_dim is a multiple of 8
   int64_t stride = p.rep_stride;
   asm volatile("" : "+s"(stride));  // (or 64 row offsets are kept across the lane's blocks, and spill)
@@ -1235,7 +1235,14 @@ __global__ __launch_bounds__(kThreads, G == 4 && LPR > 8 ? 2 : 4) void decode_ke
   if (SPLIT && p.scores) {
     if (n_ok && !bs.take_all) keys_from_scores(p, out_row, n, keys);
   } else if (n_ok && !bs.take_all) {  // (a budget that takes every block needs no scores)
-    for (int blk = tid; blk < n; blk += kThreads) keys[blk] = sel::order_key(score_block_any<G>(p, q_s, b, g, hd, blk));
+    // a whole row at head_dim 64: one round trip to memory.  With a device full
+    // of one-head lists 32 values leave registers (74, not 97) for a third
+    // resident workgroup: 96 sequences, 8/8 heads of 64, budget 16 39.3 -> 34.2 us,
+    // 200 sequences 63 -> 60 (128 of 2K tokens 40.2 -> 42.0; at 1024 lists of 8K
+    // and at 512 lists the same to 2%).
+    constexpr int kBatch = !SPLIT && G == 1 && LPR == 8 ? 32 : 64;
+    for (int blk = tid; blk < n; blk += kThreads)
+      keys[blk] = sel::order_key(score_block_any<G, kBatch>(p, q_s, b, g, hd, blk));
   }
   if (wave == kWaves - 1) cl.early[lane] = early;
   if (tid == 0) cl.late_ready = 0;
