@@ -43,7 +43,10 @@ def state(kv):
     (16, 8, 16, 1, True, 4),       # two launches: 2 query heads, representatives per query head
     (8, 8, None, 1, False, 4),     # two launches: 1 query head per KV head, no input RMSNorm
     (32, 8, None, 1, True, 4),     # 4 query heads per KV head: the two calls
-    (16, 8, None, 2, True, 4),     # split attention: the two calls
+    (16, 8, None, 2, True, 4),     # two launches, several workgroups per list
+    (16, 8, 16, 2, False, 4),      # the same, representatives per query head, no input RMSNorm
+    (8, 8, None, 2, True, 4),      # the same, 1 query head per KV head
+    (8, 8, None, 2, False, 3),     # the same, no input RMSNorm
     (16, 8, None, 1, True, 70),    # two launches over two 64-row tiles of the projection
 ])
 def test_decode_step_qkv_equals_two_calls(hip, hq, hkv, rep_heads, splits, rms, batch):
