@@ -8,9 +8,11 @@ blocks, 4 planted blocks per KV head), one token appended per layer and step.
 
 Timed two ways, each on its own copy of the same state and as HIP graphs of
 whole decode steps:
-  * one launch per layer (decode_kernel_shared: every workgroup of the
-    sequence scores the whole shared set, selects, and attends its KV head);
-  * the split launches (append + seal, score + select, attention + merge).
+  * one launch per layer (decode_step: decode_kernel_shared, every workgroup of
+    the sequence scores the whole shared set, selects, and attends its share of
+    its KV head's pages);
+  * the split launches (append + seal, scoring, selection, attention, merge: the
+    separate calls).
 Reported: µs per layer-step of each, and, on the last step, the two paths'
 ids equal, their outputs within fp32 rounding, and their states (pool,
 representatives, counters) equal bit for bit.  Parity with the oracle is in
@@ -46,19 +48,28 @@ def run(args):
     scale = float(np.float32(1.0) / np.sqrt(np.float32(D)))
     status = torch.zeros(1, dtype=torch.int32, device="cuda")
     results = {}
-    for mode, splits in (("one_launch", 1), ("split_launches", 2)):
+    for mode in ("one_launch", "split_launches"):
         L = [bench.Layer(sa, torch, cfg, l, args, total_steps) for l in range(layers)]
-        fused = sa.select_attend_fused(L[0].kv, 1, splits, sel_stride=budget)
-        assert fused == (splits == 1), (mode, fused)
-        ws, _ = sa.decode_step_workspace(L[0].kv, splits)
+        kv = L[0].kv
+        ws, _ = sa.decode_step_workspace(kv)
+        scores = torch.empty((batch, 1, kv.rep_stride), dtype=torch.float32, device="cuda")
+        records = torch.empty(sa.lib().sa_hip_attention_workspace_bytes(batch, hq, hkv, D, 2) // 4,
+                              dtype=torch.float32, device="cuda")
         sel = torch.full((layers, batch, 1, budget), -1, dtype=torch.int32, device="cuda")
         cnt = torch.zeros((layers, batch, 1), dtype=torch.int32, device="cuda")
         out = torch.empty((layers, batch, hq, D), dtype=torch.float32, device="cuda")
 
         def step(s):
             for l, ly in enumerate(L):
-                sa.decode_step(ly.kv, ly.knew[s], ly.vnew[s], 0, ly.q[s], 1, budget, init, local, scale, ws,
-                               selected=sel[l], counts=cnt[l], out=out[l], splits=splits, status=status)
+                if mode == "one_launch":
+                    sa.decode_step(ly.kv, ly.knew[s], ly.vnew[s], 0, ly.q[s], 1, budget, init, local, scale, ws,
+                                   selected=sel[l], counts=cnt[l], out=out[l], status=status)
+                    continue
+                sa.append_seal(ly.kv, ly.knew[s], ly.vnew[s], 0, status=status)
+                sa.score_select_split(ly.kv, ly.q[s], 1, budget, init, local, selected=sel[l], counts=cnt[l],
+                                      scores=scores, status=status)
+                sa.sparse_decode_attention(ly.kv, ly.q[s], sel[l], cnt[l], scale, out=out[l], splits=2,
+                                           workspace=records, status=status)
 
         for s in range(warmup):
             step(s)

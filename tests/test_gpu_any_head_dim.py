@@ -204,8 +204,9 @@ def test_attention_general_head_dim_bad_block_flagged(hip):
     (200, 8, 8, 8, 1, 3, False), (64, 32, 8, 8, 1, 0, True), (64, 16, 8, 8, 2, 0, False)])
 def test_decode_steps_general_head_dim(hip, d, hq, hkv, groups, splits, local, f16):
     """sa_hip_decode_step at another head_dim over 36 steps that seal blocks:
-    one launch (decode_kernel_rows: selection per KV group, splits 1) or its
-    launches in sequence (append + seal, scoring, selection, attention);
+    one launch (decode_kernel_rows: selection per KV group; splits > 1: several
+    workgroups per list) or, for groups of several KV heads, append + seal, a
+    scoring launch and that kernel on its scores;
     state bit-exact, ids equal, attention within 2e-3 of the oracle at every
     step, fp32 and FP16 token input."""
     print(f"case: decode steps d={d} hq={hq} hkv={hkv} groups={groups} splits={splits} f16={f16}", flush=True)

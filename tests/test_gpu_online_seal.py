@@ -91,7 +91,8 @@ def test_decode_step_online_bit_exact(hip, hq, local_tokens, ring_tokens, window
 @pytest.mark.parametrize("hq,splits", [(64, 1), (16, 2), (32, 2)])
 def test_online_seal_separate_launches(hip, hq, splits):
     """8 query heads per KV head (no fused kernel) and split requests run
-    sa_hip_append_seal_online + selection + attention: the same results."""
+    sa_hip_append_seal_online's launch, then the rest of the step in one with
+    several workgroups per list: the same results."""
     print(f"case: hq={hq} splits={splits}", flush=True)
     case = make_case(950 + hq, 2, hq, 8, [32 * 20 + 29, 32 * 7 + 31], table_stride=30, rep_heads=hq)
     kv = device_kv(case)

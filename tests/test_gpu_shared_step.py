@@ -109,7 +109,7 @@ def test_shared_decode_steps_bit_exact(hip, hq, local_tokens, f16):
 def test_c1_shape_shared_decode_steps_equal_split_launches(hip):
     """The reference's C1/C2 shape (1 sequence, 16 query / 8 KV heads, 2048
     tokens, budget 16 = init 1 + local 2 + 13): 40 one-launch steps against
-    the same steps as separate launches (splits 2) on a copy of the state:
+    the same steps as the separate calls on a copy of the state:
     ids, counts, pool, representatives and counters equal bit for bit, the
     outputs to fp32 rounding (the pages are visited in another order), and
     both within 2e-3 of the oracle."""
@@ -117,7 +117,6 @@ def test_c1_shape_shared_decode_steps_equal_split_launches(hip):
     kv_a, kv_b = device_kv(case), device_kv(case)
     assert hip.select_attend_fused(kv_a, 1) and not hip.select_attend_fused(kv_a, 1, splits=2)
     ws_a, _ = hip.decode_step_workspace(kv_a)
-    ws_b, _ = hip.decode_step_workspace(kv_b, 2)
     st = status_tensor()
     rng = np.random.default_rng(23)
     budget, init, local = 16, 1, 2
@@ -128,8 +127,9 @@ def test_c1_shape_shared_decode_steps_equal_split_launches(hip):
         q = to_dev(case.query)
         sel_a, cnt_a, out_a = hip.decode_step(kv_a, to_dev(k), to_dev(v), 0, q, 1, budget, init, local, SCALE, ws_a,
                                               status=st)
-        sel_b, cnt_b, out_b = hip.decode_step(kv_b, to_dev(k), to_dev(v), 0, q, 1, budget, init, local, SCALE, ws_b,
-                                              splits=2, status=st)
+        hip.append_seal(kv_b, to_dev(k), to_dev(v), 0, status=st)
+        sel_b, cnt_b, _ = hip.score_select_split(kv_b, q, 1, budget, init, local, status=st)
+        out_b = hip.sparse_decode_attention(kv_b, q, sel_b, cnt_b, SCALE, splits=2, status=st)
         esel, ecnt, expect = oracle_shared_decode(case, 0, budget, init, local, budget, k=k, v=v)
         torch.cuda.synchronize()
         assert int(st.item()) == 0, step

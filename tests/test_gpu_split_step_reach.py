@@ -1,8 +1,8 @@
 """GPU parity: the decode step with several workgroups per (sequence, KV head)
 at head dimensions other than 128 (lists past 1024 blocks: scores from a launch
 of their own, selection by the whole workgroup up to 4096 blocks and by one wave
-beyond; budgets that take up to 16 workgroups per list), and with per-sequence
-budgets.  State and ids bit-exact with the oracle, the attention within 2e-3."""
+beyond; budgets that take up to 16 workgroups per list; the shapes it does not
+take), and with per-sequence budgets.  State and ids bit-exact with the oracle, the attention within 2e-3."""
 import numpy as np
 import pytest
 import torch
@@ -28,6 +28,11 @@ CASES = [
     (200, 8, 8, 8, [PAGE * 135 + 30], 70),
     (64, 16, 8, 1, [PAGE * 130 + 31], 64),
     (24, 3, 3, 3, [PAGE * 300 + 31], 256),
+    # the separate launches at another head_dim: one past the row walk's, 8 query heads per KV head, and 17 KV
+    # heads at more pages than one workgroup per list is taken for
+    (320, 4, 2, 2, [PAGE * 40 + 31, PAGE * 9], 16),
+    (64, 16, 2, 2, [PAGE * 50 + 30], 20),
+    (64, 17, 17, 17, [PAGE * 90 + 31], 80),
 ]
 
 
