@@ -220,7 +220,9 @@ __global__ __launch_bounds__(kMergeThreads) void merge_partials_kernel(const Par
   }
   // The records' loads are issued kMergeBatch at a time (indices past the
   // last record read the last one and are not used); the maximum over all
-  // records comes first, then the weighted sums are added in chunk order.
+  // records comes first, then the weighted sums are added in chunk order, each
+  // batch's on its own and then to the total: one rounding of the whole sum per
+  // batch instead of one per record.
   constexpr int kMergeBatch = 8;
   for (int o = threadIdx.x; o < G * D; o += kThreads) {
     const int h = o / D;
@@ -246,13 +248,16 @@ __global__ __launch_bounds__(kMergeThreads) void merge_partials_kernel(const Par
           l[j] = rec[1];
           a[j] = rec[kPartPad + d];
         }
+        float lb = 0.0f, ab = 0.0f;
 #pragma unroll
         for (int j = 0; j < kMergeBatch; ++j) {
           if (z0 + j >= records || m[j] == kNegInf) continue;
           const float f = __builtin_amdgcn_exp2f(m[j] - mx);
-          lw = __builtin_fmaf(l[j], f, lw);
-          aw = __builtin_fmaf(a[j], f, aw);
+          lb = __builtin_fmaf(l[j], f, lb);
+          ab = __builtin_fmaf(a[j], f, ab);
         }
+        lw += lb;
+        aw += ab;
       }
     }
     p.out[(static_cast<int64_t>(b) * p.query_heads + g * G + h) * D + d] = lw > 0.0f ? aw / lw : 0.0f;

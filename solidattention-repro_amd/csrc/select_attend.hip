@@ -296,13 +296,16 @@ __device__ inline void merge_split_records(const Params& p, int b, int g, int hd
       lw *= corr;
       aw *= corr;
       mx = bm;
+      float lb = 0.0f, ab = 0.0f;  // (the batch on its own, as merge_partials_kernel)
 #pragma unroll
       for (int j = 0; j < kBatch; ++j) {
         if (z0 + j >= p.splits || m[j] == attn::kNegInf) continue;
         const float f = __builtin_amdgcn_exp2f(m[j] - mx);
-        lw = __builtin_fmaf(l[j], f, lw);
-        aw = __builtin_fmaf(a[j], f, aw);
+        lb = __builtin_fmaf(l[j], f, lb);
+        ab = __builtin_fmaf(a[j], f, ab);
       }
+      lw += lb;
+      aw += ab;
     }
     p.out[(static_cast<int64_t>(b) * p.query_heads + g * G + h) * hd + d] = lw > 0.0f ? aw / lw : 0.0f;
   }
