@@ -340,9 +340,10 @@ size_t sa_hip_decode_step_workspace_bytes(const sa_paged_kv* kv,
  * variant) runs as one launch only with select_groups == kv_heads.
  * Otherwise, with few enough sequences and short enough lists, it is still
  * one launch (behind append + seal for the online seal) with several
- * workgroups per (sequence, KV head), however many the device has room for;
- * splits only selects this form (ids and state the same, outputs to fp32
- * rounding).  Else it runs the separate launches.  The _f16 variant takes raw FP16
+ * workgroups per (sequence, KV head), however many the device has room for
+ * (ids and state the same, outputs to fp32 rounding).  Else, also where that
+ * would be fewer workgroups than splits with long walks for each, or where out
+ * overlaps query (and is not query), k or v, it runs the separate launches.  The _f16 variant takes raw FP16
  * K/V bits like sa_hip_append_seal_f16.  Replaces the reference's per-layer
  * decode sequence of append_fp16_kv (qwen_layer_main.cpp:270-281 via
  * qwen_chain_main.cpp:390-391), the tail seal (kv_lifecycle_main.cpp:92-113),
